@@ -158,6 +158,18 @@ struct Gen {
   int rank = 0, a = -1;
   bool flat = true;
   int V = 1, TPL = 1, NC = 1, WG = 256, GPW = 1, FK = 1;
+  // Lines along an axis that is not the last ("column" kernels): a work-group is CW threads across
+  // consecutive lines, V adjacent lines each, times TPL threads along the axis; every per-line
+  // value is then an array over the V lines.
+  bool col = false;
+  int CW = 1;
+  // A reduction split over Z slices of the axis: a PART kernel writes each slice's accumulators to
+  // a scratch buffer ([Z][lines] per reduction), a FOLD kernel combines them in slice order.
+  enum Mode { WHOLE, PART, FOLD } mode = WHOLE;
+  uint64_t Z = 1;
+  struct Part { uint64_t value = 0, index = 0; };  // byte offsets of a reduction's partials
+  std::map<int, Part> parts;
+  uint64_t scratch = 0;
   uint64_t lines = 1, L = 1, N = 1;
   bool idx64 = false;
   std::vector<int> param_slots;
@@ -171,6 +183,7 @@ struct Gen {
   std::vector<int> first_phase;    // per node: first phase computing it
   bool has_final = false;
   bool unroll = false;
+  bool counted = false;  // loops along the line have a trip count instead of a test per chunk
   int min_waves = 1;  // amdgpu_waves_per_eu lower bound of a line kernel
 
   Gen(const Region& r, const std::vector<Slot>& s, int i) : R(r), slots(s), index(i) {}
@@ -228,11 +241,16 @@ struct Gen {
   }
   std::string ix() const { return idx64 ? "u64" : "u32"; }
 
-  // value of node i at element j (FULL) or as a line scalar (LINE)
+  // per-line values of a column kernel are arrays over its V lines
+  bool line_arrays() const { return col && V > 1; }
+  std::string at(const std::string& name, const std::string& j) const { return line_arrays() ? name + "[" + j + "]" : name; }
+  // value of node i at element j (FULL) or as a line value (LINE)
   std::string val(int i, const std::string& j) const {
     if (full(i)) return "f" + std::to_string(i) + "[" + j + "]";
-    return "s" + std::to_string(i);
+    return at("s" + std::to_string(i), j);
   }
+  // the axis that vectors and coordinate c_expr + j run along
+  int vaxis() const { return flat || col ? rank - 1 : a; }
 
   std::string op_expr(int ni, const std::string& j) const;
   void plan_layout();
@@ -295,17 +313,31 @@ struct Gen {
   std::string aix_none() const { return L >= ((uint64_t)1 << 31) ? "(i64)9223372036854775807ll" : "(i32)2147483647"; }
   void emit_full_node(int ni, int phase, const std::string& c_expr);
   void emit_line_node(int ni);
+  void emit_line_value(int ni);
   void emit_red_init(int ni);
   void emit_red_update(int ni, const std::string& k_expr, const std::string& j);
   void emit_red_chunk_arg(int ni);
-  void emit_red_finish(int ni, int phase);
+  void emit_red_fold(int ni, int phase);
+  void emit_red_fold_col(int ni);
+  void emit_red_final(int ni);
+  std::string acc_type(int ni) const;
+  std::string comb(int ni, const std::string& ov, const std::string& j) const;
+  std::string comb_arg(int ni, const std::string& ov, const std::string& oi, const std::string& on, const std::string& j) const;
+  void plan_columns();
+  void plan_split();
+  void emit_head(const std::string& entry);
+  void emit_coords();
+  void emit_bases(bool line_leaves);
+  void emit_partials(int ni);
+  void emit_fold_kernel(const std::string& entry);
+  int scratch_param() const { return (int)param_slots.size(); }
   // A float ArgReduce over vector chunks folds per chunk: the chunk's extreme (one maxNum/minNum
   // tree), one strict comparison with the running best, and a conditional copy of the chunk's
   // values; the index inside the winning chunk is found once per thread at the end. Per element
   // that is about a third of the compare-and-select-index work of a per-element fold.
   bool chunk_arg(int ni) const {
     const RNode& n = node(ni);
-    return n.kind == (int)OpKind::ArgReduce && V >= 2 && fvalued(node(n.in[0]).dtype) && !flat;
+    return n.kind == (int)OpKind::ArgReduce && V >= 2 && fvalued(node(n.in[0]).dtype) && !flat && !col;
   }
   bool chunk_arg_packed(int ni) const { return chunk_arg(ni) && node(node(ni).in[0]).dtype == DType::BF16 && V % 2 == 0; }
   std::string leaf_base(int leaf) const;
@@ -317,8 +349,8 @@ struct Gen {
     char hex[16];
     std::snprintf(hex, sizeof hex, "%06llx", (unsigned long long)(h & 0xffffff));
     rc->entry = prefix + "_" + hex;
-    size_t at = src.find("KU_ENTRY_PLACEHOLDER");
-    src.replace(at, std::string("KU_ENTRY_PLACEHOLDER").size(), rc->entry);
+    const std::string ph = "KU_ENTRY_PLACEHOLDER";
+    for (size_t p = src.find(ph); p != std::string::npos; p = src.find(ph, p + rc->entry.size())) src.replace(p, ph.size(), rc->entry);
     return src;
   }
 };
@@ -386,7 +418,7 @@ std::string Gen::op_expr(int ni, const std::string& j) const {
       return ld(n.to, raw);
     }
     case RK_DIV:
-      if (div_by_line_recip(ni)) return "(" + in(0) + " * s" + std::to_string(n.in[1]) + "_inv)";
+      if (div_by_line_recip(ni)) return "(" + in(0) + " * " + at("s" + std::to_string(n.in[1]) + "_inv", j) + ")";
       return "(" + in(0) + " / " + in(1) + ")";
     case RK_EXP: return f64 ? "exp(" + in(0) + ")" : "expf(" + in(0) + ")";
     case RK_SQRT_ADD_EPS: {
@@ -422,10 +454,11 @@ void Gen::plan_layout() {
     if (lo < 0) maxoff = std::max<size_t>(maxoff, (size_t)1 << 40);
   }
   idx64 = maxoff >= ((size_t)1 << 31);
-  int vecaxis = flat ? rank - 1 : a;
   uint64_t inner = 1;
   if (!flat)
     for (int d = a + 1; d < rank; ++d) inner *= R.S[d];
+  col = inner > 1;
+  const int vecaxis = vaxis();
   L = flat ? R.S[rank - 1] : R.S[a];
   // lines: the iteration shape without its line axis (still counted when that axis is empty: a
   // reduction over a zero-length axis writes its identity to every line)
@@ -434,7 +467,6 @@ void Gen::plan_layout() {
     if (d != (flat ? rank - 1 : a)) lines *= R.S[d];
   // vector width: 16 bytes of the narrowest streamed type, only along a contiguous last axis
   int minw = 8;
-  bool contiguous_axis = flat || inner == 1;
   for (auto& l : R.leaves)
     if (l.view.strides[vecaxis] != 0) minw = std::min<int>(minw, (int)dt_width(l.dtype));
   // A line region's V and TPL fix the order its reductions add in, so they depend only on what
@@ -444,8 +476,9 @@ void Gen::plan_layout() {
   // size their vectors by their outputs too.
   if (flat)
     for (auto& op : R.outputs) minw = std::min<int>(minw, (int)dt_width(node(op.first).dtype));
-  V = contiguous_axis ? std::min(8, 16 / std::max(minw, 1)) : 1;
-  while (V > 1 && (L % (uint64_t)V) != 0) V /= 2;
+  V = std::min(8, 16 / std::max(minw, 1));
+  while (V > 1 && (R.S[vecaxis] % (uint64_t)V) != 0) V /= 2;
+  if (col) plan_columns();
   leaf_vec.assign(R.leaves.size(), false);
   for (size_t i = 0; i < R.leaves.size(); ++i) {
     const View& v = R.leaves[i].view;
@@ -468,14 +501,8 @@ void Gen::plan_layout() {
     FK = fk ? std::max(1, std::atoi(fk)) : 1;
     return;
   }
+  if (col) return;
   uint64_t chunks = (L + V - 1) / V;
-  if (inner > 1) {
-    TPL = 1;
-    WG = 256;
-    GPW = 256;
-    NC = (int)chunks;
-    return;
-  }
   // Chunks of 16 bytes per thread, the line cached in registers. Lines of 4-byte elements take ~8
   // per thread, measured: the f32 [8192, 32000] softmax rows 5.57-5.60 -> 5.74-5.82 TB/s (1024
   // threads per row, from 16 chunks), the f32 [4096, 4096] fused reduce 5.28 -> 5.61 TB/s (128
@@ -501,6 +528,60 @@ void Gen::plan_layout() {
   // (its cross-wave combine, barriers included, then spans the whole group)
   WG = TPL > 64 ? TPL : 256;
   GPW = WG / TPL;
+  plan_split();
+}
+
+// One level of reductions and nothing computed from them per element: the axis may be split over
+// work-groups. The rule looks at the region's structure only, not at what is stored, so a
+// reduction keeps its bits when it is evaluated with other outputs.
+static bool splittable(const Region& R) {
+  for (auto& n : R.nodes)
+    if (n.level > 1 || (n.level == 1 && n.space == Space::Full)) return false;
+  return true;
+}
+
+// Threads of a column kernel. A wave reads CW * V consecutive elements of a row, so its loads
+// coalesce; a work-group's threads along the axis fold through LDS. Before, one thread walked one
+// whole line, so a launch had `lines` threads and each a serial chain of L loads: the f32
+// [16384, 1000] column sum took 2413 us on 4 work-groups and takes 20.5 us (65.5 MB, 3.2 TB/s,
+// both launches) on 1024 work-groups of 64 x 4 threads and 256 slices. Bound by the read, the ramp
+// and drain of two short launches.
+void Gen::plan_columns() {
+  const uint64_t threads = (uint64_t)1 << 18;  // 16 waves per CU
+  const bool split = splittable(R);
+  // unsplittable regions spread over the chip by lines alone: narrower vectors, then narrower
+  // groups (16 threads still read 64-byte segments of 4-byte elements)
+  if (!split)
+    while (V > 1 && lines / V < 64 * 256) V /= 2;
+  const uint64_t nvl = (lines + V - 1) / V;
+  CW = 64;
+  while (CW > 1 && (uint64_t)CW / 2 >= nvl) CW /= 2;
+  if (!split)
+    while (CW > 16 && nvl / CW < 256) CW /= 2;
+  const int most = split ? 256 : 1024;
+  TPL = 1;
+  // at least 8 rows per thread: short lines keep one thread each and their values in registers
+  while (CW * TPL < most && L > 16 && L / (2 * TPL) >= 8 && (CW * TPL < 64 || nvl * TPL < threads)) TPL *= 2;
+  WG = std::max(64, CW * TPL);
+  CW = WG / TPL;
+  GPW = CW;
+  NC = (int)((L + TPL - 1) / TPL);
+  if (!split) return;
+  // slices: enough threads to fill the chip, at least 16 rows per thread in each
+  const uint64_t groups = (nvl + CW - 1) / CW;
+  while (groups * WG * Z < threads && L / ((uint64_t)TPL * Z * 2) >= 16 && Z < 1024) Z *= 2;
+  if (Z > 1) NC = (int)((L + TPL * Z - 1) / (TPL * Z));
+}
+
+// A few long lines: slices of 8 chunks per thread (at 1024 threads a line of up to 16 chunks each
+// stays with one work-group: the second launch costs more than it spreads).
+void Gen::plan_split() {
+  if (NC <= 16 || lines >= 256 || !splittable(R)) return;
+  const uint64_t chunks = (L + V - 1) / V;
+  TPL = WG = 256;
+  GPW = 1;
+  Z = std::min<uint64_t>((chunks + 8 * TPL - 1) / (8 * TPL), std::max<uint64_t>(1, 2048 / lines));
+  NC = (int)((chunks + TPL * Z - 1) / (TPL * Z));
 }
 
 // Phases: level p = 1..P fold reductions of level p; LINE nodes of level p follow.
@@ -580,6 +661,9 @@ void Gen::schedule() {
     // a smaller footprint than the budget allows buys more resident waves: ask for them
     if (!std::getenv("KURUMI_HIP_LINE_WAVES")) min_waves = std::max(min_waves, std::min(8, 512 / (regs + 40)));
   }
+  // loops along a column, and slices, hold nothing from one phase to the next
+  counted = !flat && cached.empty() && (col || Z > 1);
+  if (counted) unroll = false;
   // with caches, later phases need fewer recomputations: rebuild need sets
   if (!cached.empty()) {
     need.assign(nph + 2, {});
@@ -608,7 +692,7 @@ static std::string imm_expr(const Leaf& l) {
 
 std::string Gen::leaf_base(int li) const {
   const View& v = R.leaves[li].view;
-  int vecaxis = flat ? rank - 1 : a;
+  const int vecaxis = vaxis();
   std::ostringstream e;
   e << "(" << ix() << ")(" << v.offset << "ll";
   for (int d = 0; d < rank; ++d) {
@@ -624,7 +708,7 @@ void Gen::emit_leaf_load(int ni, const std::string& c_expr) {
   const RNode& n = node(ni);
   const Leaf& l = R.leaves[n.leaf];
   const View& v = l.view;
-  int vecaxis = flat ? rank - 1 : a;
+  const int vecaxis = vaxis();
   std::string T = stype(l.dtype), C = ctype(l.dtype);
   std::string P = "p" + std::to_string(slot_param.at(l.slot));
   std::string base = "b" + std::to_string(n.leaf);
@@ -718,7 +802,7 @@ void Gen::emit_full_node(int ni, int phase, const std::string& c_expr) {
     emit_leaf_load(ni, c_expr);
   } else if (n.kind == RK_PADSEL) {
     // zero outside the pad windows; the non-vector axes are tested once, the vector axis per j
-    int vecaxis = flat ? rank - 1 : a;
+    const int vecaxis = vaxis();
     std::ostringstream cond;
     cond << "true";
     for (int d = 0; d < rank; ++d) {
@@ -736,7 +820,7 @@ void Gen::emit_full_node(int ni, int phase, const std::string& c_expr) {
     o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) f" << ni << "[j] = (" << condj.str()
       << ") ? " << val(n.in[0], "j") << " : (" << ctype(n.dtype) << ")0;\n";
   } else if (n.kind == (int)OpKind::Iota || n.kind == (int)OpKind::RandUniform) {
-    int vecaxis = flat ? rank - 1 : a;
+    const int vecaxis = vaxis();
     o << "      " << ctype(n.dtype) << " f" << ni << "[" << V << "];\n";
     o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) {\n";
     if (n.kind == (int)OpKind::Iota) {
@@ -798,34 +882,77 @@ void Gen::emit_full_node(int ni, int phase, const std::string& c_expr) {
 
 void Gen::emit_line_node(int ni) {
   const RNode& n = node(ni);
+  std::string expr;
   if (n.kind == RK_LEAF) {
     const Leaf& l = R.leaves[n.leaf];
     std::string P = "p" + std::to_string(slot_param.at(l.slot));
-    std::string raw = l.imm ? imm_expr(l)
-                            : "((const " + std::string(stype(l.dtype)) + "*)" + P + ")[b" + std::to_string(n.leaf) + "]";
-    o << "  const " << ctype(n.dtype) << " s" << ni << " = " << ld(l.dtype, raw) << ";\n";
+    std::string off = "b" + std::to_string(n.leaf);
+    if (line_arrays()) off += " + (" + ix() + ")(j * " + std::to_string(l.view.strides[rank - 1]) + "ll)";
+    std::string raw = l.imm ? imm_expr(l) : "((const " + std::string(stype(l.dtype)) + "*)" + P + ")[" + off + "]";
+    expr = ld(l.dtype, raw);
   } else {
-    o << "  const " << ctype(n.dtype) << " s" << ni << " = " << op_expr(ni, "0") << ";\n";
+    expr = op_expr(ni, line_arrays() ? "j" : "0");
   }
-  if (needs_line_recip(ni)) o << "  const float s" << ni << "_inv = 1.0f / s" << ni << ";\n";
+  const std::string sn = "s" + std::to_string(ni);
+  if (line_arrays()) {
+    o << "  " << ctype(n.dtype) << " " << sn << "[" << V << "];\n  #pragma unroll\n  for (int j = 0; j < " << V << "; ++j) "
+      << sn << "[j] = " << expr << ";\n";
+  } else {
+    o << "  const " << ctype(n.dtype) << " " << sn << " = " << expr << ";\n";
+  }
+  emit_line_value(ni);
+}
+
+// A per-line value's reciprocal where one is used, and its store where it is an output.
+void Gen::emit_line_value(int ni) {
+  const RNode& n = node(ni);
+  const std::string sn = "s" + std::to_string(ni);
+  if (needs_line_recip(ni)) {
+    if (line_arrays())
+      o << "  float " << sn << "_inv[" << V << "];\n  #pragma unroll\n  for (int j = 0; j < " << V << "; ++j) " << sn
+        << "_inv[j] = 1.0f / " << sn << "[j];\n";
+    else
+      o << "  const float " << sn << "_inv = 1.0f / " << sn << ";\n";
+  }
   auto it = out_slot.find(ni);
-  if (it != out_slot.end() && !full(ni) && !flat) {
-    o << "  if (lane == 0) ((" << stype(n.dtype) << "*)p" << slot_param.at(it->second) << ")[line] = "
-      << st(n.dtype, "s" + std::to_string(ni)) << ";\n";
-  }
+  if (it == out_slot.end() || full(ni) || flat || mode == PART) return;
+  const std::string dst = "((" + std::string(stype(n.dtype)) + "*)p" + std::to_string(slot_param.at(it->second)) + ")";
+  o << "  if (lane == 0" << (col ? " && live" : "") << ") ";
+  if (line_arrays())
+    o << "{\n    #pragma unroll\n    for (int j = 0; j < " << V << "; ++j) " << dst << "[line + j] = "
+      << st(n.dtype, sn + "[j]") << ";\n  }\n";
+  else
+    o << dst << "[line] = " << st(n.dtype, sn) << ";\n";
+}
+
+// accumulator type of a reduction (ArgReduce: of its running best value)
+std::string Gen::acc_type(int ni) const {
+  const RNode& n = node(ni);
+  DType in = node(n.in[0]).dtype;
+  if (n.kind == (int)OpKind::ArgReduce) return ctype(in);
+  if (fvalued(n.dtype) || in == DType::F32) return "float";
+  if (n.dtype == DType::F64) return "double";
+  return n.kind == (int)OpKind::ReduceMax ? stype(n.dtype) : utype(n.dtype);
 }
 
 void Gen::emit_red_init(int ni) {
   const RNode& n = node(ni);
   DType in = node(n.in[0]).dtype;
-  std::string r = std::to_string(ni);
+  std::string r = std::to_string(ni), A = acc_type(ni);
+  const std::string dim = line_arrays() ? "[" + std::to_string(V) + "]" : "";
+  auto decl = [&](const std::string& type, const std::string& name, const std::string& init) {
+    if (dim.empty()) o << "  " << type << " " << name << " = " << init << ";\n";
+    else o << "  " << type << " " << name << dim << ";\n  #pragma unroll\n  for (int j = 0; j < " << V << "; ++j) " << name
+           << "[j] = " << init << ";\n";
+  };
   if (n.kind == (int)OpKind::ArgReduce) {
     bool mx = n.arg == ArgKind::Max;
     std::string init;
     if (fvalued(in) || in == DType::F64) init = flt_lit(in == DType::F64 ? DType::F64 : DType::F32, mx ? -INFINITY : INFINITY);
     else init = mx ? int_min(in) : int_max(in);
-    o << "  " << ctype(in) << " bv" << r << " = " << init << "; " << aix() << " bi" << r << " = " << aix_none()
-      << "; bool bn" << r << " = false;\n";
+    decl(A, "bv" + r, init);
+    decl(aix(), "bi" + r, aix_none());
+    decl("bool", "bn" + r, "false");
     if (chunk_arg(ni)) {
       // the winning chunk: its first element index and its values (bf16 values two to a word)
       o << "  " << aix() << " bc" << r << " = " << aix_none() << "; ";
@@ -834,16 +961,11 @@ void Gen::emit_red_init(int ni) {
     }
     return;
   }
-  DType acc = n.dtype;
-  std::string A;
-  if (fvalued(acc) || in == DType::F32) A = "float";
-  else if (acc == DType::F64) A = "double";
-  else A = n.kind == (int)OpKind::ReduceMax ? stype(acc) : utype(acc);
   std::string init;
   if (n.kind == (int)OpKind::Sum) init = "(" + A + ")0";
   else if (n.kind == (int)OpKind::Prod) init = "(" + A + ")1";
-  else init = (A == "float" || A == "double") ? flt_lit(A == "double" ? DType::F64 : DType::F32, -INFINITY) : int_min(acc);
-  o << "  " << A << " acc" << r << " = " << init << ";\n";
+  else init = (A == "float" || A == "double") ? flt_lit(A == "double" ? DType::F64 : DType::F32, -INFINITY) : int_min(n.dtype);
+  decl(A, "acc" + r, init);
 }
 
 void Gen::emit_red_update(int ni, const std::string& k_expr, const std::string& j) {
@@ -858,23 +980,25 @@ void Gen::emit_red_update(int ni, const std::string& k_expr, const std::string& 
     // keeps the first index of equal values; NaN never compares true and is skipped. The
     // reference's NaN-at-index-0 rule (the result is 0) is a flag set by the element k == 0.
     std::string k = "((" + aix() + ")(" + k_expr + "))";
-    o << "        { " << ctype(in) << " v_ = " << v << "; if (v_ " << cmp << " bv" << r << ") { bv" << r
-      << " = v_; bi" << r << " = " << k << "; }";
-    if (fvalued(in) || in == DType::F64) o << " if (" << j << " == 0 && " << k << " == 0 && v_ != v_) bn" << r << " = true;";
+    o << "        { " << ctype(in) << " v_ = " << v << "; if (v_ " << cmp << " " << at("bv" + r, j) << ") { " << at("bv" + r, j)
+      << " = v_; " << at("bi" + r, j) << " = " << k << "; }";
+    if (fvalued(in) || in == DType::F64)
+      o << " if (" << (col ? "" : j + " == 0 && ") << k << " == 0 && v_ != v_) " << at("bn" + r, j) << " = true;";
     o << " }\n";
     return;
   }
+  const std::string acc = at("acc" + r, j);
   bool fl = fvalued(n.dtype) || n.dtype == DType::F64 || in == DType::F32;
   if (n.kind == (int)OpKind::Sum) {
-    if (fl) o << "        acc" << r << " += " << v << ";\n";
-    else o << "        acc" << r << " = acc" << r << " + (" << utype(n.dtype) << ")" << v << ";\n";
+    if (fl) o << "        " << acc << " += " << v << ";\n";
+    else o << "        " << acc << " = " << acc << " + (" << utype(n.dtype) << ")" << v << ";\n";
   } else if (n.kind == (int)OpKind::Prod) {
-    if (fl) o << "        acc" << r << " *= " << v << ";\n";
-    else o << "        acc" << r << " = acc" << r << " * (" << utype(n.dtype) << ")" << v << ";\n";
+    if (fl) o << "        " << acc << " *= " << v << ";\n";
+    else o << "        " << acc << " = " << acc << " * (" << utype(n.dtype) << ")" << v << ";\n";
   } else {
-    if (n.dtype == DType::F64) o << "        acc" << r << " = fmax(acc" << r << ", " << v << ");\n";
-    else if (fl) o << "        acc" << r << " = fmaxf(acc" << r << ", " << v << ");\n";
-    else o << "        acc" << r << " = (" << v << " > acc" << r << ") ? " << v << " : acc" << r << ";\n";
+    if (n.dtype == DType::F64) o << "        " << acc << " = fmax(" << acc << ", " << v << ");\n";
+    else if (fl) o << "        " << acc << " = fmaxf(" << acc << ", " << v << ");\n";
+    else o << "        " << acc << " = (" << v << " > " << acc << ") ? " << v << " : " << acc << ";\n";
   }
 }
 
@@ -902,25 +1026,76 @@ void Gen::emit_red_chunk_arg(int ni) {
   o << "      }\n";
 }
 
+// One more partial of an ArgReduce into its running best: the better value, the smaller index of
+// equal ones, never a NaN; the NaN-at-index-0 flag accumulates.
+std::string Gen::comb_arg(int ni, const std::string& ov, const std::string& oi, const std::string& on, const std::string& j) const {
+  const RNode& n = node(ni);
+  DType in = node(n.in[0]).dtype;
+  const std::string r = std::to_string(ni), bv = at("bv" + r, j), bi = at("bi" + r, j), bn = at("bn" + r, j);
+  std::string cmp = n.arg == ArgKind::Max ? ">" : "<";
+  std::string ok = (fvalued(in) || in == DType::F64) ? "(" + ov + " == " + ov + ") && " : "";
+  return "{ if (" + ok + "(" + ov + " " + cmp + " " + bv + " || (" + ov + " == " + bv + " && " + oi + " < " + bi +
+         "))) { " + bv + " = " + ov + "; " + bi + " = " + oi + "; } " + bn + " = " + bn + " || " + on + "; }";
+}
+
+// One more partial of any other reduction into its accumulator.
+std::string Gen::comb(int ni, const std::string& ov, const std::string& j) const {
+  const RNode& n = node(ni);
+  DType in = node(n.in[0]).dtype;
+  const std::string acc = at("acc" + std::to_string(ni), j);
+  if (n.kind == (int)OpKind::Sum) return acc + " = " + acc + " + " + ov + ";";
+  if (n.kind == (int)OpKind::Prod) return acc + " = " + acc + " * " + ov + ";";
+  if (n.dtype == DType::F64) return acc + " = fmax(" + acc + ", " + ov + ");";
+  if (fvalued(n.dtype) || in == DType::F32) return acc + " = fmaxf(" + acc + ", " + ov + ");";
+  return acc + " = (" + ov + " > " + acc + ") ? " + ov + " : " + acc + ";";
+}
+
+// Fold across the TPL threads of a column kernel's lines: a tree through LDS (one buffer for all
+// reductions, lds_red), the totals read back by every thread.
+void Gen::emit_red_fold_col(int ni) {
+  if (TPL == 1) return;
+  const RNode& n = node(ni);
+  const bool arg = n.kind == (int)OpKind::ArgReduce;
+  const std::string r = std::to_string(ni), A = acc_type(ni), I = aix(), none = aix_none();
+  const std::string head = "    #pragma unroll\n    for (int j = 0; j < " + std::to_string(V) + "; ++j) ";
+  const std::string w = std::to_string(WG), me = "[j * " + w + " + threadIdx.x]";
+  o << "  {\n    " << A << "* lv = (" << A << "*)lds_red;\n";
+  // the flag travels in the index: -1 (no index is negative)
+  if (arg) o << "    " << I << "* li = (" << I << "*)(lds_red + " << (uint64_t)WG * V << ");\n";
+  o << "    __syncthreads();\n";
+  auto put = [&] {
+    if (arg) o << head << "{ lv" << me << " = " << at("bv" + r, "j") << "; li" << me << " = " << at("bn" + r, "j") << " ? (" << I
+               << ")-1 : " << at("bi" + r, "j") << "; }\n";
+    else o << head << "lv" << me << " = " << at("acc" + r, "j") << ";\n";
+  };
+  put();
+  o << "    __syncthreads();\n    #pragma unroll 1\n    for (int s_ = " << TPL / 2 << "; s_ >= 1; s_ >>= 1) {\n      if (lane < (u32)s_) {\n";
+  const std::string other = "[j * " + w + " + threadIdx.x + s_ * " + std::to_string(CW) + "]";
+  if (arg)
+    o << head << "{ " << A << " ov = lv" << other << "; " << I << " oi = li" << other << "; bool on = oi < 0; "
+      << comb_arg(ni, "ov", "oi", "on", "j") << " }\n";
+  else
+    o << head << "{ " << A << " ov = lv" << other << "; " << comb(ni, "ov", "j") << " }\n";
+  put();
+  o << "      }\n      __syncthreads();\n    }\n";
+  const std::string top = "[j * " + w + " + threadIdx.x % " + std::to_string(CW) + "]";
+  if (arg)
+    o << head << "{ " << at("bv" + r, "j") << " = lv" << top << "; " << at("bi" + r, "j") << " = li" << top << "; "
+      << at("bn" + r, "j") << " = li" << top << " < 0; }\n";
+  else
+    o << head << at("acc" + r, "j") << " = lv" << top << ";\n";
+  o << "  }\n";
+}
+
 // cross-lane fold of a reduction (butterfly within the wave, LDS across waves)
-void Gen::emit_red_finish(int ni, int phase) {
+void Gen::emit_red_fold(int ni, int phase) {
+  if (col) return emit_red_fold_col(ni);
   const RNode& n = node(ni);
   std::string r = std::to_string(ni);
   bool arg = n.kind == (int)OpKind::ArgReduce;
   DType in = node(n.in[0]).dtype;
-  auto comb_arg = [&](const std::string& ov, const std::string& oi, const std::string& on) {
-    std::string cmp = n.arg == ArgKind::Max ? ">" : "<";
-    std::string ok = (fvalued(in) || in == DType::F64) ? "(" + ov + " == " + ov + ") && " : "";
-    return "{ if (" + ok + "(" + ov + " " + cmp + " bv" + r + " || (" + ov + " == bv" + r + " && " + oi + " < bi" + r +
-           "))) { bv" + r + " = " + ov + "; bi" + r + " = " + oi + "; } bn" + r + " = bn" + r + " || " + on + "; }";
-  };
-  auto comb = [&](const std::string& ov) {
-    if (n.kind == (int)OpKind::Sum) return "acc" + r + " = acc" + r + " + " + ov + ";";
-    if (n.kind == (int)OpKind::Prod) return "acc" + r + " = acc" + r + " * " + ov + ";";
-    if (n.dtype == DType::F64) return "acc" + r + " = fmax(acc" + r + ", " + ov + ");";
-    if (fvalued(n.dtype) || in == DType::F32) return "acc" + r + " = fmaxf(acc" + r + ", " + ov + ");";
-    return "acc" + r + " = (" + ov + " > acc" + r + ") ? " + ov + " : acc" + r + ";";
-  };
+  auto comb_arg = [&](const std::string& ov, const std::string& oi, const std::string& on) { return this->comb_arg(ni, ov, oi, on, "0"); };
+  auto comb = [&](const std::string& ov) { return this->comb(ni, ov, "0"); };
   if (chunk_arg(ni)) {
     // the index of the first element of the winning chunk equal to the best value
     o << "  if (bc" << r << " != " << aix_none() << ") {\n    " << aix() << " bj_ = " << V - 1 << ";\n";
@@ -967,22 +1142,143 @@ void Gen::emit_red_finish(int ni, int phase) {
       o << "  for (int w = 1; w < " << W << "; ++w) { auto ov = lr" << tag << "[w]; " << comb("ov") << " }\n";
     }
   }
-  // final value
-  if (arg) {
-    o << "  const i64 s" << r << " = (bn" << r << " || bi" << r << " == " << aix_none() << ") ? 0ll : (i64)bi" << r
-      << ";\n";
+}
+
+// The reduction's final value s<r> (rounded to its dtype), stored where it is an output.
+void Gen::emit_red_final(int ni) {
+  const RNode& n = node(ni);
+  const std::string r = std::to_string(ni);
+  auto value = [&](const std::string& j) {
+    if (n.kind == (int)OpKind::ArgReduce)
+      return "(" + at("bn" + r, j) + " || " + at("bi" + r, j) + " == " + aix_none() + ") ? 0ll : (i64)" + at("bi" + r, j);
+    std::string v = at("acc" + r, j);
+    return dt_is_int(n.dtype) ? std::string("(") + stype(n.dtype) + ")" + v : rnd(n.dtype, v);
+  };
+  const std::string T = n.kind == (int)OpKind::ArgReduce ? "i64" : ctype(n.dtype);
+  if (line_arrays())
+    o << "  " << T << " s" << r << "[" << V << "];\n  #pragma unroll\n  for (int j = 0; j < " << V << "; ++j) s" << r
+      << "[j] = " << value("j") << ";\n";
+  else
+    o << "  const " << T << " s" << r << " = " << value("0") << ";\n";
+  emit_line_value(ni);
+}
+
+// A PART kernel's accumulators of its slice, one row of the reduction's [Z][lines] partials.
+void Gen::emit_partials(int ni) {
+  const std::string r = std::to_string(ni), A = acc_type(ni), I = aix();
+  const bool arg = node(ni).kind == (int)OpKind::ArgReduce;
+  const Part& pt = parts.at(ni);
+  const std::string head = line_arrays() ? "    #pragma unroll\n    for (int j = 0; j < " + std::to_string(V) + "; ++j) " : "    ";
+  const std::string where = "[(u64)z * " + std::to_string(lines) + "ull + line" + (line_arrays() ? " + j]" : "]");
+  o << "  if (lane == 0" << (col ? " && live" : "") << ") {\n";
+  o << head << "((" << A << "*)(ps + " << pt.value << "ull))" << where << " = " << at(arg ? "bv" + r : "acc" + r, "j") << ";\n";
+  if (arg)
+    o << head << "((" << I << "*)(ps + " << pt.index << "ull))" << where << " = " << at("bn" + r, "j") << " ? (" << I << ")-1 : "
+      << at("bi" + r, "j") << ";\n";
+  o << "  }\n";
+}
+
+// Kernel signature: leaves, outputs, then (split reductions) the partials.
+void Gen::emit_head(const std::string& entry) {
+  o << "extern \"C\" __global__ void __launch_bounds__(" << WG << ") ";
+  // line kernels: ask for the occupancy the cache budget was sized for (two groups per CU)
+  if (!flat && min_waves > 1 && !counted) o << "__attribute__((amdgpu_waves_per_eu(" << min_waves << "))) ";
+  o << entry << "(";
+  for (size_t i = 0; i < param_slots.size(); ++i) o << (i ? ", " : "") << "void* __restrict__ p" << i;
+  if (mode != WHOLE) o << (param_slots.empty() ? "" : ", ") << "u8* __restrict__ ps";
+  o << ") {\n";
+}
+
+// Which line, thread along it and slice this thread works on, and the line's coordinates.
+void Gen::emit_coords() {
+  if (col) {
+    const uint64_t nvl = lines / V, groups = (nvl + CW - 1) / CW;
+    o << "  const u32 lane = threadIdx.x / " << CW << "u;\n";
+    o << "  const u64 vl_ = (u64)(blockIdx.x % " << groups << "u) * " << CW << "ull + threadIdx.x % " << CW << "u;\n";
+    if (nvl % CW) o << "  const bool live = vl_ < " << nvl << "ull;\n";  // the others repeat the last line, unstored
+    else o << "  constexpr bool live = true;\n";
+    o << "  const u64 line = (live ? vl_ : " << nvl - 1 << "ull) * " << V << "ull;\n";
+    if (mode == PART) o << "  const u32 z = blockIdx.x / " << groups << "u;\n";
+    uint64_t lds = 0;  // 8-byte words of the shared fold buffer
+    for (auto& n : R.nodes)
+      if (is_red(n.kind)) lds = std::max<uint64_t>(lds, (uint64_t)WG * V * (n.kind == (int)OpKind::ArgReduce ? 2 : 1));
+    if (TPL > 1) o << "  __shared__ u64 lds_red[" << lds << "];\n";
   } else {
-    std::string v = "acc" + r;
-    if (dt_is_int(n.dtype)) v = std::string("(") + stype(n.dtype) + ")" + v;
-    else v = rnd(n.dtype, v);
-    o << "  const " << ctype(n.dtype) << " s" << r << " = " << v << ";\n";
-    if (needs_line_recip(ni)) o << "  const float s" << r << "_inv = 1.0f / s" << r << ";\n";
+    o << "  const u32 lane = threadIdx.x % " << TPL << "u;\n";
+    if (mode == PART) {
+      o << "  const u64 line = blockIdx.x / " << Z << "u;\n  const u32 z = blockIdx.x % " << Z << "u;\n";
+    } else {
+      o << "  const u64 line = (u64)blockIdx.x * " << GPW << "ull + threadIdx.x / " << TPL << "u;\n";
+      if ((uint64_t)GPW * (((lines + GPW - 1) / GPW)) != lines) o << "  if (line >= " << lines << "ull) return;\n";
+    }
   }
-  auto it = out_slot.find(ni);
-  if (it != out_slot.end()) {
-    o << "  if (lane == 0) ((" << stype(n.dtype) << "*)p" << slot_param.at(it->second) << ")[line] = "
-      << st(n.dtype, "s" + r) << ";\n";
+  o << "  " << ix() << " t = (" << ix() << ")line;\n";
+  for (int d = rank - 1; d >= 0; --d) {
+    if (d == a) continue;
+    o << "  const " << ix() << " c" << d << " = t % " << R.S[d] << "u; t /= " << R.S[d] << "u;\n";
   }
+  o << "  (void)t;\n";
+}
+
+// Leaf bases (+ padding validity on the non-vector axes). A column kernel's line leaves have
+// theirs ahead of the loop along the axis, the others inside it, where c<axis> is known.
+void Gen::emit_bases(bool line_leaves) {
+  const int vecaxis = vaxis();
+  for (size_t li = 0; li < R.leaves.size(); ++li) {
+    const View& v = R.leaves[li].view;
+    if (col && (v.strides[a] == 0 && !v.padded()) != line_leaves) continue;
+    // b<leaf> is the element index modulo the index width: a padded view's offset may lie before
+    // the buffer, so the vector-axis term is always added in the index type before the pointer
+    o << "  const " << ix() << " b" << li << " = " << leaf_base((int)li);
+    if (col && line_leaves && v.strides[rank - 1]) o << " + (" << ix() << ")((i64)c" << rank - 1 << " * " << v.strides[rank - 1] << "ll)";
+    o << ";\n";
+    if (v.padded()) {
+      o << "  const bool vb" << li << " = true";
+      for (int d = 0; d < rank; ++d) {
+        if (d == vecaxis) continue;
+        if (v.wlo[d] > 0) o << " && (i64)c" << d << " >= " << v.wlo[d];
+        if (v.whi[d] < (int64_t)v.shape[d]) o << " && (i64)c" << d << " < " << v.whi[d];
+      }
+      o << ";\n";
+    }
+  }
+}
+
+// FOLD: the slices' accumulators combined in slice order, then everything that follows the
+// reductions. One line per thread across, as in a column kernel.
+void Gen::emit_fold_kernel(const std::string& entry) {
+  mode = FOLD;
+  col = true;
+  V = 1;
+  CW = 64;
+  while (CW > 1 && (uint64_t)CW / 2 >= lines) CW /= 2;
+  TPL = 1;
+  while (CW * TPL < 256 && (uint64_t)TPL * 2 <= Z) TPL *= 2;
+  WG = std::max(64, CW * TPL);
+  CW = WG / TPL;
+  emit_head(entry);
+  emit_coords();
+  emit_bases(true);
+  for (size_t i = 0; i < R.nodes.size(); ++i)
+    if (!full((int)i) && node((int)i).level == 0 && !is_red(node((int)i).kind)) emit_line_node((int)i);
+  for (auto& kv : parts) {
+    const int r = kv.first;
+    const bool arg = node(r).kind == (int)OpKind::ArgReduce;
+    emit_red_init(r);
+    const std::string A = acc_type(r), I = aix(), where = "[(u64)z * " + std::to_string(lines) + "ull + line]";
+    o << "  #pragma unroll 8\n  for (u32 z = lane; z < " << Z << "u; z += " << TPL << "u) { const " << A << " ov = ((const " << A
+      << "*)(ps + " << kv.second.value << "ull))" << where << "; ";
+    if (arg)
+      o << "const " << I << " oi = ((const " << I << "*)(ps + " << kv.second.index << "ull))" << where << "; const bool on = oi < 0; "
+        << comb_arg(r, "ov", "oi", "on", "0") << " }\n";
+    else
+      o << comb(r, "ov", "0") << " }\n";
+    emit_red_fold(r, 1);
+    emit_red_final(r);
+  }
+  for (size_t i = 0; i < R.nodes.size(); ++i)
+    if (!full((int)i) && node((int)i).level == 1 && !is_red(node((int)i).kind)) emit_line_node((int)i);
+  o << "}\n";
 }
 
 std::string Gen::generate(RegionCode* rc) {
@@ -998,14 +1294,21 @@ std::string Gen::generate(RegionCode* rc) {
   for (auto& l : R.leaves) param(l.slot);
   for (auto& op : R.outputs) param(op.second);
   o << kDevicePrelude;
-  o << "extern \"C\" __global__ void __launch_bounds__(" << WG << ") ";
-  // line kernels: ask for the occupancy the cache budget was sized for (two groups per CU)
-  if (!flat && min_waves > 1) o << "__attribute__((amdgpu_waves_per_eu(" << min_waves << "))) ";
-  o << entry << "(";
-  for (size_t i = 0; i < param_slots.size(); ++i) o << (i ? ", " : "") << "void* __restrict__ p" << i;
-  o << ") {\n";
-  int vecaxis = flat ? rank - 1 : a;
-  std::vector<int> lines_leaves;
+  if (Z > 1) {
+    mode = PART;
+    auto room = [&](size_t width) {
+      const uint64_t at = scratch;
+      scratch = (scratch + Z * lines * width + 255) / 256 * 256;
+      return at;
+    };
+    for (size_t i = 0; i < R.nodes.size(); ++i)
+      if (is_red(R.nodes[i].kind)) {
+        Part& pt = parts[(int)i];
+        pt.value = room(8);
+        if (R.nodes[i].kind == (int)OpKind::ArgReduce) pt.index = room(8);
+      }
+  }
+  emit_head(entry);
   if (flat) {
     // FK chunks per thread, each a block-wide coalesced stripe, unrolled so their loads are in
     // flight together
@@ -1020,32 +1323,9 @@ std::string Gen::generate(RegionCode* rc) {
     }
     o << "  (void)t;\n";
   } else {
-    o << "  const u32 lane = threadIdx.x % " << TPL << "u;\n";
-    o << "  const u64 line = (u64)blockIdx.x * " << GPW << "ull + threadIdx.x / " << TPL << "u;\n";
-    if ((uint64_t)GPW * (((lines + GPW - 1) / GPW)) != lines) o << "  if (line >= " << lines << "ull) return;\n";
-    o << "  " << ix() << " t = (" << ix() << ")line;\n";
-    for (int d = rank - 1; d >= 0; --d) {
-      if (d == a) continue;
-      o << "  const " << ix() << " c" << d << " = t % " << R.S[d] << "u; t /= " << R.S[d] << "u;\n";
-    }
-    o << "  (void)t;\n";
+    emit_coords();
   }
-  // leaf bases (+ padding validity on the non-vector axes)
-  for (size_t li = 0; li < R.leaves.size(); ++li) {
-    // b<leaf> is the element index modulo the index width: a padded view's offset may lie before
-    // the buffer, so the vector-axis term is always added in the index type before the pointer
-    o << "  const " << ix() << " b" << li << " = " << leaf_base((int)li) << ";\n";
-    const View& v = R.leaves[li].view;
-    if (v.padded()) {
-      o << "  const bool vb" << li << " = true";
-      for (int d = 0; d < rank; ++d) {
-        if (d == vecaxis) continue;
-        if (v.wlo[d] > 0) o << " && (i64)c" << d << " >= " << v.wlo[d];
-        if (v.whi[d] < (int64_t)v.shape[d]) o << " && (i64)c" << d << " < " << v.whi[d];
-      }
-      o << ";\n";
-    }
-  }
+  emit_bases(true);
   if (flat) {
     // single pass over V elements
     std::string cexpr = "c" + std::to_string(rank - 1);
@@ -1103,14 +1383,37 @@ std::string Gen::generate(RegionCode* rc) {
       if (is_red(node((int)i).kind) && node((int)i).level == p) reds.push_back((int)i);
     for (int r : reds) emit_red_init(r);
     // chunk loop
-    if (unroll) o << "  #pragma unroll\n";
-    else o << "  #pragma unroll 2\n";
-    o << "  for (int c = 0; c < " << NC << "; ++c) {\n";
-    o << "    const u32 ch = (u32)c * " << TPL << "u + lane;\n";
-    bool guard = (uint64_t)NC * TPL * V != L;
-    if (guard) o << "    if ((u64)ch * " << V << "ull < " << L << "ull) {\n";
-    else o << "    {\n";
-    std::string cexpr = "ch * " + std::to_string(V) + "u";
+    std::string cexpr, kexpr;
+    if (col) {
+      cexpr = "c" + std::to_string(rank - 1);
+      kexpr = "c" + std::to_string(a);
+    } else {
+      cexpr = "ch * " + std::to_string(V) + "u";
+      kexpr = cexpr + " + j";
+    }
+    // this thread's chunks: positions first + c * TPL of the line's `total`
+    const uint64_t total = col ? L : (L + V - 1) / V;
+    const std::string pos = mode == PART ? "((u64)z * " + std::to_string(NC) + "ull + c) * " + std::to_string(TPL) + "ull + lane"
+                                         : "(u64)c * " + std::to_string(TPL) + "ull + lane";
+    const std::string idt = col ? ix() : "u32", idn = col ? kexpr : "ch";
+    if (counted) {
+      // a trip count instead of a test per chunk, so that the unrolled loads go out together
+      const std::string first = mode == PART ? "(u64)z * " + std::to_string((uint64_t)NC * TPL) + "ull + lane" : "(u64)lane";
+      o << "  const u64 first" << p << " = " << first << ";\n";
+      o << "  const int nc" << p << " = first" << p << " >= " << total << "ull ? 0 : (int)min((u64)" << NC << ", (" << total - 1
+        << "ull - first" << p << ") / " << TPL << "ull + 1);\n";
+      o << "  #pragma unroll " << std::max(4, std::min(16, 32 / V)) << "\n";
+      o << "  for (int c = 0; c < nc" << p << "; ++c) {\n    const " << idt << " " << idn << " = (" << idt << ")(" << pos << ");\n    {\n";
+    } else {
+      if (unroll) o << "  #pragma unroll\n";
+      else o << "  #pragma unroll 2\n";
+      o << "  for (int c = 0; c < " << NC << "; ++c) {\n";
+      o << "    const " << idt << " " << idn << " = (" << idt << ")c * " << TPL << "u + lane;\n";
+      bool guard = (uint64_t)NC * TPL != total;
+      if (guard) o << "    if ((u64)" << idn << " < " << total << "ull) {\n";
+      else o << "    {\n";
+    }
+    if (col) emit_bases(false);
     for (size_t i = 0; i < R.nodes.size(); ++i)
       if (need[p].count((int)i)) emit_full_node((int)i, p, cexpr);
     for (int r : reds) {
@@ -1119,7 +1422,7 @@ std::string Gen::generate(RegionCode* rc) {
         continue;
       }
       o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) {\n";
-      emit_red_update(r, "ch * " + std::to_string(V) + "u + j", "j");
+      emit_red_update(r, kexpr, "j");
       o << "      }\n";
     }
     // FULL outputs stored in this phase
@@ -1132,9 +1435,10 @@ std::string Gen::generate(RegionCode* rc) {
       std::ostringstream ob;
       ob << "(" << ix() << ")(0";
       for (int d = 0; d < rank; ++d)
-        if (d != a) ob << " + (" << ix() << ")c" << d << " * " << rs[d] << "u";
+        if (d != vaxis()) ob << " + (" << ix() << ")c" << d << " * " << rs[d] << "u";
       ob << ")";
-      if (V > 1 && rs[a] == 1) {
+      if (col) o << "      if (live) {\n";
+      if (V > 1 && rs[vaxis()] == 1) {
         const bool nts = nt_mode() & 1;
         if (n.dtype == DType::BF16 && V % 2 == 0 && full(op.first)) {
           // every bf16 value is carried bf16-exact in f32: its pattern is the upper half
@@ -1150,19 +1454,32 @@ std::string Gen::generate(RegionCode* rc) {
         }
       } else {
         o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) ((" << T << "*)" << Pp << ")["
-          << ob.str() << " + ((" << ix() << ")(" << cexpr << ") + j) * " << rs[a] << "u] = "
+          << ob.str() << " + ((" << ix() << ")(" << cexpr << ") + j) * " << rs[vaxis()] << "u] = "
           << st(n.dtype, val(op.first, "j")) << ";\n";
       }
+      if (col) o << "      }\n";
     }
     o << "    }\n  }\n";
-    for (int r : reds) emit_red_finish(r, p);
+    for (int r : reds) emit_red_fold(r, p);
+    if (mode == PART) {
+      for (int r : reds) emit_partials(r);
+      break;
+    }
+    for (int r : reds) emit_red_final(r);
     for (size_t i = 0; i < R.nodes.size(); ++i)
       if (!full((int)i) && node((int)i).level == p && !is_red(node((int)i).kind)) emit_line_node((int)i);
   }
   o << "}\n";
-  rc->grid = (unsigned)((lines + GPW - 1) / GPW);
+  const uint64_t units = col ? lines / V : lines, per = col ? CW : GPW;
+  rc->grid = (unsigned)((units + per - 1) / per * Z);
   rc->block = WG;
   rc->arg_slots = param_slots;
+  if (mode == PART) {
+    emit_fold_kernel(entry + "_fold");
+    rc->scratch_bytes = scratch;
+    rc->fold_grid = (unsigned)((lines + CW - 1) / CW);
+    rc->fold_block = WG;
+  }
   return finish(prefix, rc);
 }
 

@@ -1795,6 +1795,15 @@ void Plan::compile() {
       s.label = rc.entry;
       sources_.push_back(rc.src);
       if (ctx_) s.fn = ctx_->modules().get(rc.src, rc.entry);
+      if (rc.scratch_bytes) {
+        Slot scratch;
+        scratch.bytes = rc.scratch_bytes;
+        slots_.push_back(std::move(scratch));
+        s.arg_slots.push_back((int)slots_.size() - 1);
+        s.fold_grid = rc.fold_grid;
+        s.fold_block = rc.fold_block;
+        if (ctx_) KU_HIP(hipModuleGetFunction(&s.fold_fn, s.fn.mod, (rc.entry + "_fold").c_str()));
+      }
     } else if (s.type == Step::GEMM) {
       const GemmStep& G = gemms_[s.index];
       GemmArgs a;
@@ -1876,6 +1885,7 @@ void Plan::launch_step(const Step& s) {
     }
     if (s.grid == 0) return;
     KU_HIP(hipModuleLaunchKernel(s.fn.fn, s.grid, 1, 1, s.block, 1, 1, 0, st, args.data(), nullptr));
+    if (s.fold_fn) KU_HIP(hipModuleLaunchKernel(s.fold_fn, s.fold_grid, 1, 1, s.fold_block, 1, 1, 0, st, args.data(), nullptr));
     ctx_->profile().launches[(int)Kind::Fused]++;
   } else if (s.type == Step::GEMM) {
     const GemmStep& G = gemms_[s.index];

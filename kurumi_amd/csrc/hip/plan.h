@@ -158,6 +158,8 @@ struct Step {
   KernelFn fn;
   unsigned grid = 0, block = 0;
   std::vector<int> arg_slots;
+  hipFunction_t fold_fn = nullptr;  // split reductions: the second kernel
+  unsigned fold_grid = 0, fold_block = 0;
   std::string label;
 };
 
@@ -281,6 +283,10 @@ struct RegionCode {
   std::string src, entry;
   unsigned grid = 0, block = 0;
   std::vector<int> arg_slots;  // leaf/output slots in kernel parameter order
+  // a reduction split over slices of its axis: partials of `scratch_bytes` go through one more
+  // buffer (the last parameter of both kernels) to the kernel <entry>_fold of the same source
+  size_t scratch_bytes = 0;
+  unsigned fold_grid = 0, fold_block = 0;
 };
 RegionCode gen_region(const Region& r, const std::vector<Slot>& slots, int index);
 
