@@ -27,6 +27,9 @@ struct GemmArgs {
   // optional fused cast: the (scaled) f32 result is first rounded to this 16-bit float type (the
   // contraction's own dtype, GT_BF16 / GT_F16), then converted to out_type; -1: no extra rounding
   int round_type = -1;
+  // gemm_scratch_bytes() of device memory for a K split's partial sums; with less, K is not split
+  void* ws = nullptr;
+  size_t ws_bytes = 0;
 };
 
 // Compute units of the current device (cached on first use): sizes persistent grids and tile rounds.
@@ -34,8 +37,11 @@ int cu_count();
 
 // Short name of the kernel variant that will run (for plan labels): the MFMA kernel's element
 // type, layout and tile ("gemm_mfma_bf16_nn_256x256"; "_a64" when an operand spans 2^31 bytes or
-// more and the 64-bit-address DMA form runs), or "gemm_generic".
+// more and the 64-bit-address DMA form runs), the
+// register-staged kernel's "gemm_mfma_<type>_<layout>_<tile>_flex[_split<n>]", or "gemm_generic".
 std::string gemm_variant(const GemmArgs& a);
+// scratch that the variant uses (0 for most); `a.a` / `a.b` need the alignment of the operands only
+size_t gemm_scratch_bytes(const GemmArgs& a);
 void launch_gemm(const GemmArgs& a, hipStream_t s);
 
 struct AttnArgs {

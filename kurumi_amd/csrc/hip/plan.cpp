@@ -1796,21 +1796,19 @@ void Plan::compile() {
       sources_.push_back(rc.src);
       if (ctx_) s.fn = ctx_->modules().get(rc.src, rc.entry);
       if (rc.scratch_bytes) {
-        Slot scratch;
-        scratch.bytes = rc.scratch_bytes;
-        slots_.push_back(std::move(scratch));
-        s.arg_slots.push_back((int)slots_.size() - 1);
+        s.arg_slots.push_back(scratch_slot(rc.scratch_bytes));
         s.fold_grid = rc.fold_grid;
         s.fold_block = rc.fold_block;
         if (ctx_) KU_HIP(hipModuleGetFunction(&s.fold_fn, s.fn.mod, (rc.entry + "_fold").c_str()));
       }
     } else if (s.type == Step::GEMM) {
-      const GemmStep& G = gemms_[s.index];
-      GemmArgs a;
-      a.sab = G.sab; a.sam = G.sam; a.sak = G.sak; a.sbb = G.sbb; a.sbk = G.sbk; a.sbn = G.sbn;
-      a.batch = (int64_t)G.batch; a.m = (int64_t)G.m; a.n = (int64_t)G.n; a.k = (int64_t)G.k;
-      a.in_type = (int)G.in_dtype; a.out_type = (int)G.out_dtype;
+      GemmStep& G = gemms_[s.index];
+      GemmArgs a = gemm_args(G);
+      // what the launch will see of the operands' addresses: buffers are 256-byte aligned
+      a.a = reinterpret_cast<const char*>(256) + G.a_off * (int64_t)dt_width(G.in_dtype);
+      a.b = reinterpret_cast<const char*>(256) + G.b_off * (int64_t)dt_width(G.in_dtype);
       if (G.alpha_slot >= 0) a.alpha = reinterpret_cast<const float*>(16);
+      G.ws_slot = scratch_slot(gemm_scratch_bytes(a));
       std::ostringstream o;
       o << gemm_variant(a) << " b" << G.batch << " m" << G.m << " n" << G.n << " k" << G.k;
       if (G.out_dtype != G.in_dtype && G.alpha_slot < 0) o << " +cast " << dt_name(G.out_dtype);
@@ -1821,7 +1819,13 @@ void Plan::compile() {
       o << "actq_e4m3 " << dt_name(A.x_dtype) << " n" << A.n;
       s.label = o.str();
     } else if (s.type == Step::QUANT) {
-      const QuantStep& Q = quants_[s.index];
+      QuantStep& Q = quants_[s.index];
+      if (Q.path == QuantStep::DEQUANT_GEMM) {
+        GemmArgs a = quant_gemm_args(Q);
+        a.a = reinterpret_cast<const char*>(256) + Q.act_off * (int64_t)dt_width(Q.act_dtype);
+        a.b = reinterpret_cast<const char*>(256);
+        Q.ws_slot = scratch_slot(gemm_scratch_bytes(a));
+      }
       std::ostringstream o;
       o << (Q.path == QuantStep::GEMV ? "quant_gemv" : Q.path == QuantStep::MFMA ? "quant_mfma" : "quant_dequant+gemm")
         << " int" << Q.bits << (Q.sym ? "s" : "a") << " g"
@@ -1836,6 +1840,37 @@ void Plan::compile() {
       s.label = o.str();
     }
   }
+}
+
+// A scratch buffer of the plan for one of its steps; -1 where none is needed.
+int Plan::scratch_slot(size_t bytes) {
+  if (!bytes) return -1;
+  Slot s;
+  s.dtype = DType::U8;
+  s.bytes = bytes;
+  slots_.push_back(std::move(s));
+  return (int)slots_.size() - 1;
+}
+
+// A step's GEMM without its addresses.
+GemmArgs Plan::gemm_args(const GemmStep& G) const {
+  GemmArgs a;
+  a.sab = G.sab; a.sam = G.sam; a.sak = G.sak; a.sbb = G.sbb; a.sbk = G.sbk; a.sbn = G.sbn;
+  a.batch = (int64_t)G.batch; a.m = (int64_t)G.m; a.n = (int64_t)G.n; a.k = (int64_t)G.k;
+  a.in_type = (int)G.in_dtype;
+  a.out_type = (int)G.out_dtype;
+  a.round_type = G.round_dtype == DType::BF16 || G.round_dtype == DType::F16 ? (int)G.round_dtype : -1;
+  return a;
+}
+
+// The product after a dequantisation: B[k][n] = wdq[n][k], the NT layout.
+GemmArgs Plan::quant_gemm_args(const QuantStep& Q) const {
+  GemmArgs g;
+  g.sam = (int64_t)Q.k; g.sak = 1; g.sab = 0;
+  g.sbn = (int64_t)Q.k; g.sbk = 1; g.sbb = 0;
+  g.batch = 1; g.m = (int64_t)Q.m; g.n = (int64_t)Q.n; g.k = (int64_t)Q.k;
+  g.in_type = (int)Q.wdq_dtype; g.out_type = (int)Q.act_dtype;
+  return g;
 }
 
 void Plan::allocate() {
@@ -1889,16 +1924,15 @@ void Plan::launch_step(const Step& s) {
     ctx_->profile().launches[(int)Kind::Fused]++;
   } else if (s.type == Step::GEMM) {
     const GemmStep& G = gemms_[s.index];
-    GemmArgs a;
+    GemmArgs a = gemm_args(G);
     size_t iw = dt_width(G.in_dtype);
     a.a = static_cast<const char*>(slot_ptr(slots_, G.a_slot)) + G.a_off * (int64_t)iw;
     a.b = static_cast<const char*>(slot_ptr(slots_, G.b_slot)) + G.b_off * (int64_t)iw;
     a.c = slot_ptr(slots_, G.c_slot);
-    a.sab = G.sab; a.sam = G.sam; a.sak = G.sak; a.sbb = G.sbb; a.sbk = G.sbk; a.sbn = G.sbn;
-    a.batch = (int64_t)G.batch; a.m = (int64_t)G.m; a.n = (int64_t)G.n; a.k = (int64_t)G.k;
-    a.in_type = (int)G.in_dtype;
-    a.out_type = (int)G.out_dtype;
-    a.round_type = G.round_dtype == DType::BF16 || G.round_dtype == DType::F16 ? (int)G.round_dtype : -1;
+    if (G.ws_slot >= 0) {
+      a.ws = slot_ptr(slots_, G.ws_slot);
+      a.ws_bytes = slots_[G.ws_slot].bytes;
+    }
     if (G.alpha_slot >= 0) a.alpha = static_cast<const float*>(slot_ptr(slots_, G.alpha_slot)) + G.alpha_off;
     if (G.col_scale_slot >= 0) {
       a.col_scale = static_cast<const float*>(slot_ptr(slots_, G.col_scale_slot)) + G.col_scale_off;
@@ -1950,12 +1984,12 @@ void Plan::launch_step(const Step& s) {
       a.wdq = slot_ptr(slots_, Q.wdq_slot);
       launch_quant_dequant(a, st);
       KU_HIP(hipGetLastError());
-      GemmArgs g;
+      GemmArgs g = quant_gemm_args(Q);
       g.a = a.act; g.b = a.wdq; g.c = a.out;
-      g.sam = (int64_t)Q.k; g.sak = 1; g.sab = 0;
-      g.sbn = (int64_t)Q.k; g.sbk = 1; g.sbb = 0;  // B[k][n] = wdq[n][k]: the NT layout
-      g.batch = 1; g.m = a.m; g.n = a.n; g.k = a.k;
-      g.in_type = (int)Q.wdq_dtype; g.out_type = (int)Q.act_dtype;
+      if (Q.ws_slot >= 0) {
+        g.ws = slot_ptr(slots_, Q.ws_slot);
+        g.ws_bytes = slots_[Q.ws_slot].bytes;
+      }
       launch_gemm(g, st);
     }
     KU_HIP(hipGetLastError());

@@ -17,6 +17,7 @@
 
 #include "../ir/graph.h"
 #include "../ir/tensor.h"
+#include "kernels/kernels.h"
 #include "runtime.h"
 
 namespace ku::hipbk {
@@ -114,7 +115,7 @@ struct GemmStep {
   // fused cast epilogue: round to round_dtype (the dot's bf16 / f16) before storing out_dtype;
   // F32 = no extra rounding
   DType round_dtype = DType::F32;
-  std::string variant;
+  int ws_slot = -1;  // scratch of a split K
 };
 
 // Weight-only quantized matmul: a fused dequant GEMV (M <= 8), the fused dequant MFMA kernel
@@ -132,6 +133,7 @@ struct QuantStep {
   DType act_dtype = DType::BF16, wdq_dtype = DType::BF16;
   bool tile_const = false;
   const void* qw_tiled = nullptr;
+  int ws_slot = -1;  // scratch of the GEMM after a dequantisation
 };
 
 struct AttnStep {
@@ -212,6 +214,9 @@ class Plan {
  private:
   friend class Planner;
   void compile();
+  int scratch_slot(size_t bytes);
+  GemmArgs gemm_args(const GemmStep& G) const;
+  GemmArgs quant_gemm_args(const QuantStep& Q) const;
   void allocate();
   // device buffers of the slots, the constants from the cache and their lane-ordered copies
   void bind_device_buffers(const Graph& g, ConstCache* consts);

@@ -1,0 +1,84 @@
+"""The register-staged MFMA GEMM (f32 operands, 16-bit operands of any alignment, split K) against
+the oracle, bit for bit: operands are multiples of 1/16 in [-1, 1], so every partial sum of up to
+2^16 products is a multiple of 1/256 below 2^16 and exact in f32 in any order."""
+import numpy as np
+import pytest
+
+import kurumi_amd as K
+from kurumi_amd import DType, Tensor
+from kutest import f32_to_bf16_bits, interpret, to_f32
+
+pytestmark = pytest.mark.gpu
+
+
+def tensor(v, dt):
+    v = np.ascontiguousarray(v, np.float32)
+    if dt == DType.BF16:
+        return Tensor(dt, v.shape, f32_to_bf16_bits(v).tobytes())
+    return Tensor(dt, v.shape, (v.astype(np.float16) if dt == DType.F16 else v).tobytes())
+
+
+def sixteenths(rng, shape):
+    return rng.integers(-16, 17, shape) / np.float32(16)
+
+
+# tiles cut by M, N and K, one element, one column, rows of odd length, whole tiles, long K on few
+# tiles (split), more rows than one tile of each height
+SIZES = [(1, 1, 1), (2, 3, 5), (33, 1, 70), (1, 130, 129), (31, 65, 127), (64, 64, 64), (130, 129, 33), (7, 128, 2496),
+         (257, 300, 95), (5, 7, 9001), (200, 120, 1111)]
+
+
+@pytest.mark.parametrize("m,n,k", SIZES)
+@pytest.mark.parametrize("nt", [False, True])
+@pytest.mark.parametrize("dt", [DType.F32, DType.BF16, DType.F16])
+def test_products_of_any_size_match_oracle(hip, dt, nt, m, n, k):
+    print(f"{dt.name} nt={nt} {m}x{n}x{k}", flush=True)
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    g = K.Graph()
+    a, b = g.input([m, k], dt), g.input([n, k] if nt else [k, n], dt)
+    y = g.dot_general(a, b, [1], [1 if nt else 0])
+    feeds = {a: tensor(sixteenths(rng, (m, k)), dt), b: tensor(sixteenths(rng, (n, k) if nt else (k, n)), dt)}
+    assert "gemm_mfma" in hip.plan(g, [y], feeds).steps()[-1]
+    roots = [y, g.cast(y, DType.F16 if dt != DType.F16 else DType.F32)]
+    for r in roots:  # each alone: the cast rides in the product's epilogue
+        np.testing.assert_array_equal(hip.eval_with(g, r, feeds).numpy(), interpret(g, [r], feeds)[0].numpy())
+
+
+@pytest.mark.parametrize("dt", [DType.F32, DType.BF16])
+def test_strided_batched_and_offset_operands_match_oracle(hip, dt):
+    """Views the planner hands to the kernel as they are: a sliced operand (its rows start at any
+    element), a batch broadcast to a stride of zero, a batch of transposed right operands, and
+    reversed rows (a negative row stride)."""
+    rng = np.random.default_rng(11)
+    g = K.Graph()
+    a, b = g.input([3, 50, 83], dt), g.input([3, 83, 45], dt)
+    w, bt = g.input([83, 45], dt), g.input([3, 45, 83], dt)
+    feeds = {n: tensor(sixteenths(rng, g.shape(n)), dt) for n in (a, b, w, bt)}
+    sa = g.slice(a, [(0, 3), (1, 50), (3, 80)])
+    sb = g.slice(b, [(0, 3), (3, 80), (2, 44)])
+    roots = [g.dot_general(sa, sb, [2], [1], [0], [0]),
+             g.dot_general(a, g.broadcast_to(w, [3, 83, 45]), [2], [1], [0], [0]),
+             g.dot_general(a, bt, [2], [2], [0], [0]),
+             g.dot_general(g.flip(a, [1]), b, [2], [1], [0], [0]),
+             g.dot_general(g.slice(a, [(1, 2), (0, 50), (0, 83)]), g.slice(bt, [(2, 3), (0, 45), (0, 83)]), [2], [2], [0], [0])]
+    for i, r in enumerate(roots):
+        print(f"{dt.name} view {i}", flush=True)
+        np.testing.assert_array_equal(hip.eval_with(g, r, feeds).numpy(), interpret(g, [r], feeds)[0].numpy(), err_msg=str(i))
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 5, 7), (2, 3, 3001)])
+def test_f32_products_keep_infinities_nans_and_denormals(hip, m, n, k):
+    """Zeros stand in for what lies past K: an infinity or NaN elsewhere must not meet them, and
+    f32 denormals are neither flushed on the way in nor out."""
+    a, b = np.zeros((m, k), np.float32), np.ones((k, n), np.float32)
+    a[0, k - 1] = np.inf
+    a[1, 0] = np.float32(1e-41)
+    b[:, n - 1] = 2.0
+    b[k // 2, 1] = np.nan
+    g = K.Graph()
+    x, w = g.input([m, k], DType.F32), g.input([k, n], DType.F32)
+    got = to_f32(hip.eval_with(g, g.matmul(x, w), {x: tensor(a, DType.F32), w: tensor(b, DType.F32)}))
+    want = np.zeros((m, n), np.float32)
+    want[0], want[1], want[1, n - 1] = np.inf, np.float32(1e-41), np.float32(1e-41) * 2
+    want[:, 1] = np.nan
+    np.testing.assert_array_equal(got, want)
