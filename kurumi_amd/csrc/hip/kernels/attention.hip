@@ -16,6 +16,8 @@ namespace ku::hipbk {
 
 void launch_attention_mfma(const AttnArgs& a, hipStream_t s);
 bool attention_mfma_ok(const AttnArgs& a);
+void launch_attention_f32(const AttnArgs& a, hipStream_t s);
+bool attention_f32_ok(const AttnArgs& a);
 
 namespace {
 
@@ -76,6 +78,7 @@ bool attn_supported(const AttnArgs& a) {
 
 const char* attn_variant(const AttnArgs& a) {
   if (attention_mfma_ok(a)) return "attn_mfma";
+  if (attention_f32_ok(a)) return "attn_mfma_f32";
   return "attn_rowwise";
 }
 
@@ -83,6 +86,10 @@ void launch_attention(const AttnArgs& a, hipStream_t s) {
   if (!attn_supported(a)) throw std::runtime_error("kurumi_hip attention: unsupported shape");
   if (attention_mfma_ok(a)) {
     launch_attention_mfma(a, s);
+    return;
+  }
+  if (attention_f32_ok(a)) {
+    launch_attention_f32(a, s);
     return;
   }
   switch (a.d) {

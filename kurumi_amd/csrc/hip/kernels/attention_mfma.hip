@@ -1,7 +1,7 @@
 // Flash attention forward on MFMA for gfx950 (kernel family 4).
 //
 // out[h] = softmax(scale * q[h] k[h]^T [+ causal -inf above the diagonal]) v[h] for each of the
-// bh heads of contiguous [bh, s, d] bf16/f16 tensors: the semantics of `Op::Sdpa`
+// bh heads of contiguous [bh, s, d] bf16/f16 tensors (d 32, 64 or 128): the semantics of `Op::Sdpa`
 // (kurumi_core/src/interp/nn.rs:125-172) and of the decomposed chain
 // (graph/ops/nn/attention.rs:97-113), computed the flash way (scores never leave registers).
 //
@@ -82,6 +82,18 @@ __device__ __forceinline__ float sum2(uint32_t pair, float c) {
   }
 }
 
+// the two values of a packed pair
+template <int DT>
+__device__ __forceinline__ float lower(uint32_t pair) {
+  if constexpr (DT == GT_BF16) return __uint_as_float(pair << 16);
+  else return (float)__builtin_bit_cast(f16x2, pair)[0];
+}
+template <int DT>
+__device__ __forceinline__ float upper(uint32_t pair) {
+  if constexpr (DT == GT_BF16) return __uint_as_float(pair & 0xffff0000u);
+  else return (float)__builtin_bit_cast(f16x2, pair)[1];
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, uint32_t bytes) {
   // dword3 0x00020000: 32-bit data format, the raw-buffer setting for gfx9 parts
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
@@ -132,6 +144,12 @@ attn_mfma_k(AttnArgs a) {
   constexpr int NBLK = TBYTES / 1024 / NW;  // 1 KB DMA blocks per wave per tile
   constexpr int DS = D / 16;             // k-steps of S^T
   constexpr int DTL = D / 32;            // 32-row tiles of O^T
+  // Heads of 32 keep the probabilities to 32-bit precision: a 16-bit value plus the 16-bit value of
+  // what its rounding left (2^-17 of a probability in bf16), a product each, and f32 row sums. The
+  // P.V product is a small part of a block there: bf16 [4, 4, 2986, 32]
+  // takes 51 us (45 without the remainders, at 1.35 times the error against f64), 2876 us on the
+  // one-query-per-thread kernel.
+  constexpr bool SPLIT_P = D == 32;
   static_assert(W >= 1 && NBLK * NW * 1024 == TBYTES, "K / V staging");
   // every block a wave needs starts at or before the wave's first query, so a lane is never
   // fully masked in a block it needs
@@ -278,6 +296,7 @@ attn_mfma_k(AttnArgs a) {
     dma(vp, vc ? C.head : N.head, vc ? C.nkv : N.nkv, vc ? kb + 1 : kb + 1 - C.nkb, vbuf(P ^ 1), true);
     const int k0 = kb * BK;
     u32x4 pf[QT][4];
+    [[maybe_unused]] u32x4 pl[4];  // SPLIT_P: what the rounding to 16 bits left
 #pragma unroll
     for (int u = 0; u < QT; ++u) {
       // mask keys past the sequence and (causal) keys after the query: key k0 + off(t, v) + 4h
@@ -336,6 +355,9 @@ attn_mfma_k(AttnArgs a) {
       // the row sum adds the rounded probabilities (the ones the P.V product uses), two at a
       // time with v_dot2 against (1, 1), in two chains
       float rs[2] = {0.f, 0.f};
+      // SPLIT_P in f16: probabilities times 2^7 (at most 2^15 with the lazy maximum), so that the
+      // remainders of all but the smallest are normal f16 numbers; the row sum carries the factor too
+      const float em = (SPLIT_P && DT == GT_F16 ? 7.f : 0.f) - mc[0];
       u32x4 kf[3];
       kf[0] = kread(0);
       kf[1] = kread(1);
@@ -345,10 +367,15 @@ attn_mfma_k(AttnArgs a) {
 #pragma unroll
         for (int e = 0; e < PPM; ++e) {
           const int i = m * PPM + e, te = i >> 3, v2 = i & 7;
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[0][te][2 * v2], c, -mc[0]));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[0][te][2 * v2 + 1], c, -mc[0]));
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[0][te][2 * v2], c, em));
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[0][te][2 * v2 + 1], c, em));
           const uint32_t pp = pack2<DT>(p0, p1);
-          rs[v2 & 1] = sum2<DT>(pp, rs[v2 & 1]);
+          if constexpr (SPLIT_P) {
+            rs[v2 & 1] += p0 + p1;
+            pl[2 * te + (v2 >> 2)][v2 & 3] = pack2<DT>(p0 - lower<DT>(pp), p1 - upper<DT>(pp));
+          } else {
+            rs[v2 & 1] = sum2<DT>(pp, rs[v2 & 1]);
+          }
           // step s = 2t + v2/4 takes v = 8*(s%2) .. +7 of tile t
           pf[0][2 * te + (v2 >> 2)][v2 & 3] = pp;
         }
@@ -380,6 +407,7 @@ attn_mfma_k(AttnArgs a) {
         const u32x4 vf = u32x4{half[0][0], half[0][1], half[1][0], half[1][1]};
 #pragma unroll
         for (int u = 0; u < QT; ++u) o[u][t] = mfma<DT>(vf, pf[u][s], o[u][t]);
+        if constexpr (SPLIT_P) o[0][t] = mfma<DT>(vf, pl[s], o[0][t]);
       }
     // the S^T just issued was this tile's last: the Q fragments now belong to the next tile
     if (kb + 2 == C.nkb) load_q(N);
@@ -417,30 +445,33 @@ attn_mfma_k(AttnArgs a) {
     // swizzled by row) so every store writes whole 128-byte lines: eight rows of 16 lanes x 16
     // bytes per instruction instead of 8-byte pieces of 32 rows, whose drain through the memory
     // pipeline stalled the next tile's first instructions.
-    static_assert(QT == 1 && DTL % 2 == 0, "epilogue staging");
+    static_assert(QT == 1 && (DTL == 1 || DTL % 2 == 0), "epilogue staging");
     {
+      // dims staged at a time (64, or all 32), as rows of CR 16-byte chunks, RI rows an instruction
+      constexpr int TT = DTL == 1 ? 1 : 2, CR = TT * 4, RI = 64 / CR;
+
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l[0]), __float_as_uint(l[0]), false, false);
       const float inv = 1.f / (__uint_as_float(sw[0]) + __uint_as_float(sw[1]));
       KU_LDS unsigned char* R = vbuf(1) + wave * 4096;
       uint16_t* Oh = static_cast<uint16_t*>(a.o) + C.head * HS;
 #pragma unroll
-      for (int hf = 0; hf < DTL / 2; ++hf) {
+      for (int hf = 0; hf < DTL / TT; ++hf) {
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             // lane (qc, h) holds dims 32t + 8g + 4h .. +3 of query qc: chunk 4tt + g, bytes 8h..
-            const f32x16& ot = o[0][2 * hf + tt];
+            const f32x16& ot = o[0][TT * hf + tt];
             u32x2 w;
             w[0] = pack2<DT>(ot[4 * g] * inv, ot[4 * g + 1] * inv);
             w[1] = pack2<DT>(ot[4 * g + 2] * inv, ot[4 * g + 3] * inv);
-            *(KU_LDS u32x2*)(R + qc * 128 + (((4 * tt + g) ^ (qc & 7)) << 4) + 8 * h) = w;
+            *(KU_LDS u32x2*)(R + qc * CR * 16 + (((4 * tt + g) ^ (qc & (CR - 1))) << 4) + 8 * h) = w;
           }
         // one wave writes and reads its own region: its LDS operations complete in order
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int qr = (lane >> 3) + 8 * i, cc = lane & 7;
-          const u32x4 val = *(const KU_LDS u32x4*)(R + qr * 128 + ((cc ^ (qr & 7)) << 4));
+        for (int i = 0; i < 32 / RI; ++i) {
+          const int qr = lane / CR + RI * i, cc = lane % CR;
+          const u32x4 val = *(const KU_LDS u32x4*)(R + qr * CR * 16 + ((cc ^ (qr & (CR - 1))) << 4));
           if (qw + qr < S) *reinterpret_cast<u32x4*>(Oh + (int64_t)(qw + qr) * D + hf * 64 + cc * 8) = val;
         }
       }
@@ -475,7 +506,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 bool attention_mfma_ok(const AttnArgs& a) {
   if (const char* e = std::getenv("KURUMI_HIP_NO_MFMA"); e && *e && *e != '0') return false;
   if (!(a.dtype == GT_BF16 || a.dtype == GT_F16)) return false;
-  if (!(a.d == 64 || a.d == 128)) return false;
+  if (!(a.d == 32 || a.d == 64 || a.d == 128)) return false;
   if (a.s <= 0 || a.bh <= 0 || a.bh * ((a.s + 127) / 128) > 0x7fffffff) return false;
   if (a.s * a.d * 2 >= (int64_t(1) << 31)) return false;  // per-head buffer offsets are 32-bit
   if (a.q && (!aligned16(a.q) || !aligned16(a.k) || !aligned16(a.v) || !aligned16(a.o))) return false;
@@ -486,10 +517,12 @@ void launch_attention_mfma(const AttnArgs& a, hipStream_t s) {
   if (!attention_mfma_ok(a)) throw std::runtime_error("kurumi_hip attention: shape not supported by the MFMA kernel");
   if (a.dtype == GT_BF16) {
     if (a.d == 128) launch_d<128, GT_BF16>(a, s);
-    else launch_d<64, GT_BF16>(a, s);
+    else if (a.d == 64) launch_d<64, GT_BF16>(a, s);
+    else launch_d<32, GT_BF16>(a, s);
   } else {
     if (a.d == 128) launch_d<128, GT_F16>(a, s);
-    else launch_d<64, GT_F16>(a, s);
+    else if (a.d == 64) launch_d<64, GT_F16>(a, s);
+    else launch_d<32, GT_F16>(a, s);
   }
 }
 
