@@ -175,6 +175,22 @@ struct Gen {
   std::vector<int> param_slots;
   std::map<int, int> slot_param;
   std::vector<bool> leaf_vec;
+  std::vector<bool> leaf_odd;  // vector leaves whose rows start at any element
+  // Rows whose length is no multiple of V: the last `rem` elements go one to a thread, through the
+  // loop body emitted a second time with V = 1 (`tail`), its caches named cachet<node>.
+  uint64_t rem = 0;
+  bool tail = false, odd_out = false;
+  int mainV = 1;
+  std::string cache_name(int c) const { return (tail ? "cachet" : "cache") + std::to_string(c); }
+  // a vector load / store of `type` at `ptr`
+  std::string vload(const std::string& type, const std::string& ptr, bool nt, bool odd, size_t width) const {
+    if (odd) return "vld_at<" + type + ", " + std::to_string(width) + ", " + (nt ? "true" : "false") + ">(" + ptr + ")";
+    return (nt ? "vld_nt((const " : "*((const ") + type + "*)(" + ptr + "))";
+  }
+  std::string vstore(const std::string& type, const std::string& ptr, bool nt, bool odd, size_t width) const {
+    if (odd) return "vst_at<" + type + ", " + std::to_string(width) + ", " + (nt ? "true" : "false") + ">(" + ptr + ", w)";
+    return nt ? "vst_nt((" + type + "*)(" + ptr + "), w)" : "*(" + type + "*)(" + ptr + ") = w";
+  }
   int P = 0;  // reduction levels
   std::vector<int> store_phase;    // per node: phase in which a FULL output is stored (0 none)
   std::map<int, int> out_slot;     // rnode -> slot
@@ -294,7 +310,7 @@ struct Gen {
   // a vectorised bf16 leaf is loaded and kept as packed 32-bit words
   bool bf16_words(int c) const {
     const RNode& cn = node(c);
-    return cn.kind == RK_LEAF && R.leaves[cn.leaf].dtype == DType::BF16 && V % 2 == 0 && leaf_vec[cn.leaf] &&
+    return cn.kind == RK_LEAF && R.leaves[cn.leaf].dtype == DType::BF16 && V % 2 == 0 && leaf_vec[cn.leaf] && !tail &&
            !R.leaves[cn.leaf].view.padded() && !R.leaves[cn.leaf].imm;
   }
   // 16-bit leaves are cached two to a 32-bit register. (bf16 intermediates could be too -- every
@@ -477,9 +493,17 @@ void Gen::plan_layout() {
   if (flat)
     for (auto& op : R.outputs) minw = std::min<int>(minw, (int)dt_width(node(op.first).dtype));
   V = std::min(8, 16 / std::max(minw, 1));
-  while (V > 1 && (R.S[vecaxis] % (uint64_t)V) != 0) V /= 2;
+  // Long rows keep whole vectors at any length: the accesses need element alignment only, and the
+  // few elements left over take one more step (f32 [4, 50257] softmax + argmax, element by element
+  // from memory in every phase: 31.5 us; here 15.4 us, which is the arithmetic of one row on one CU).
+  // Short rows would gain nothing.
+  const bool any_length = !flat && !col && L >= 256;
+  while (V > 1 && !any_length && (R.S[vecaxis] % (uint64_t)V) != 0) V /= 2;
+  if (any_length) rem = L % (uint64_t)V;
+  mainV = V;
   if (col) plan_columns();
   leaf_vec.assign(R.leaves.size(), false);
+  leaf_odd.assign(R.leaves.size(), false);
   for (size_t i = 0; i < R.leaves.size(); ++i) {
     const View& v = R.leaves[i].view;
     // a padded view vectorises when its window on the vector axis is whole vectors (each
@@ -488,6 +512,7 @@ void Gen::plan_layout() {
     bool ok = V > 1 && v.strides[vecaxis] == 1 && win_ok && (v.offset % V) == 0;
     for (int d = 0; ok && d < rank; ++d)
       if (d != vecaxis && (v.strides[d] % V) != 0) ok = false;
+    if (!ok && any_length && V > 1 && v.strides[vecaxis] == 1 && !v.padded()) ok = leaf_odd[i] = true;
     leaf_vec[i] = ok;
   }
   if (flat) {
@@ -502,7 +527,7 @@ void Gen::plan_layout() {
     return;
   }
   if (col) return;
-  uint64_t chunks = (L + V - 1) / V;
+  uint64_t chunks = L / V;  // whole ones: all but `rem` elements
   // Chunks of 16 bytes per thread, the line cached in registers. Lines of 4-byte elements take ~8
   // per thread, measured: the f32 [8192, 32000] softmax rows 5.57-5.60 -> 5.74-5.82 TB/s (1024
   // threads per row, from 16 chunks), the f32 [4096, 4096] fused reduce 5.28 -> 5.61 TB/s (128
@@ -577,7 +602,7 @@ void Gen::plan_columns() {
 // stays with one work-group: the second launch costs more than it spreads).
 void Gen::plan_split() {
   if (NC <= 16 || lines >= 256 || !splittable(R)) return;
-  const uint64_t chunks = (L + V - 1) / V;
+  const uint64_t chunks = L / V;
   TPL = WG = 256;
   GPW = 1;
   Z = std::min<uint64_t>((chunks + 8 * TPL - 1) / (8 * TPL), std::max<uint64_t>(1, 2048 / lines));
@@ -626,7 +651,8 @@ void Gen::schedule() {
     // Register budget: keep at least two work-groups resident per CU (a line kernel's phases
     // are load-bound then ALU/store-bound, so a second line in flight overlaps them). With
     // W waves per group that is W/2 waves per SIMD out of 512 VGPRs, minus ~28 for the rest.
-    int waves_per_simd = std::max(1, WG / 128);
+    // Launches of at most one group per CU have no second one to keep room for.
+    int waves_per_simd = std::max(1, ((lines + GPW - 1) / GPW <= 256 ? WG / 256 : WG / 128));
     int limit = std::min(256, (512 / waves_per_simd) / 8 * 8);
     min_waves = waves_per_simd;
     if (const char* e = std::getenv("KURUMI_HIP_LINE_WAVES")) min_waves = std::atoi(e);
@@ -723,9 +749,9 @@ void Gen::emit_leaf_load(int ni, const std::string& c_expr) {
     // low half shifted up or its high half masked
     const bool ntl = flat ? (flat_nt() & 2) != 0 : (nt_mode() & 2) != 0;
     o << "      u32 rw" << ni << "[" << V / 2 << "];\n";
-    o << "      { VecT<u32, " << V / 2 << "> raw = " << (ntl ? "vld_nt(" : "*(") << "(const VecT<u32, " << V / 2
-      << ">*)((const " << T << "*)" << P << " + (" << ix() << ")(" << base << " + (" << ix() << ")(" << c_expr
-      << "))));\n";
+    const std::string VT = "VecT<u32, " + std::to_string(V / 2) + ">";
+    const std::string at = "(const " + T + "*)" + P + " + (" + ix() + ")(" + base + " + (" + ix() + ")(" + c_expr + "))";
+    o << "      { " << VT << " raw = " << vload(VT, at, ntl, leaf_odd[n.leaf], dt_width(l.dtype)) << ";\n";
     o << "        #pragma unroll\n        for (int jj = 0; jj < " << V / 2 << "; ++jj) rw" << ni << "[jj] = raw.v[jj]; }\n";
     o << "      float f" << ni << "[" << V << "];\n";
     o << "      #pragma unroll\n      for (int jj = 0; jj < " << V / 2 << "; ++jj) { f" << ni
@@ -735,7 +761,7 @@ void Gen::emit_leaf_load(int ni, const std::string& c_expr) {
   }
   // r<ni>: the stored bits (what a leaf cache keeps), f<ni>: the compute values
   o << "      " << T << " r" << ni << "[" << V << "];\n";
-  if (leaf_vec[n.leaf] && v.padded()) {
+  if (leaf_vec[n.leaf] && !tail && v.padded()) {
     std::string coord = "((i64)(" + c_expr + "))";
     o << "      if (vb" << n.leaf << " && " << coord << " >= " << v.wlo[vecaxis] << " && " << coord << " < "
       << v.whi[vecaxis] << ") { VecT<" << T << ", " << V << "> raw = *((const VecT<" << T << ", " << V
@@ -744,11 +770,11 @@ void Gen::emit_leaf_load(int ni, const std::string& c_expr) {
     o << "        #pragma unroll\n        for (int j = 0; j < " << V << "; ++j) r" << ni << "[j] = raw.v[j];\n";
     o << "      } else {\n        #pragma unroll\n        for (int j = 0; j < " << V << "; ++j) r" << ni << "[j] = ("
       << T << ")0;\n      }\n";
-  } else if (leaf_vec[n.leaf]) {
+  } else if (leaf_vec[n.leaf] && !tail) {
     const bool ntl = flat ? (flat_nt() & 2) != 0 : (nt_mode() & 2) != 0;
-    o << "      { VecT<" << T << ", " << V << "> raw = " << (ntl ? "vld_nt(" : "*(") << "(const VecT<" << T << ", " << V
-      << ">*)((const " << T << "*)" << P << " + (" << ix() << ")(" << base << " + (" << ix() << ")(" << c_expr
-      << "))));\n";
+    const std::string VT = "VecT<" + T + ", " + std::to_string(V) + ">";
+    const std::string at = "(const " + T + "*)" + P + " + (" + ix() + ")(" + base + " + (" + ix() + ")(" + c_expr + "))";
+    o << "      { " << VT << " raw = " << vload(VT, at, ntl, leaf_odd[n.leaf], dt_width(l.dtype)) << ";\n";
     o << "        #pragma unroll\n        for (int j = 0; j < " << V << "; ++j) r" << ni << "[j] = raw.v[j]; }\n";
   } else {
     int64_t sa = v.strides[vecaxis];
@@ -783,18 +809,18 @@ void Gen::emit_full_node(int ni, int phase, const std::string& c_expr) {
       // bf16 pairs to f32 without unpacking to 16-bit values: low half << 16, high half masked
       o << "      float f" << ni << "[" << V << "];\n";
       o << "      #pragma unroll\n      for (int jj = 0; jj < " << V / 2 << "; ++jj) { f" << ni
-        << "[2 * jj] = __uint_as_float(cache" << ni << "[c][jj] << 16); f" << ni << "[2 * jj + 1] = __uint_as_float(cache"
-        << ni << "[c][jj] & 0xffff0000u); }\n";
+        << "[2 * jj] = __uint_as_float(" << cache_name(ni) << "[c][jj] << 16); f" << ni << "[2 * jj + 1] = __uint_as_float("
+        << cache_name(ni) << "[c][jj] & 0xffff0000u); }\n";
     } else if (packed_cache(ni)) {
       o << "      " << stype(R.leaves[n.leaf].dtype) << " r" << ni << "[" << V << "];\n";
-      o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) r" << ni << "[j] = (u16)(cache" << ni
+      o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) r" << ni << "[j] = (u16)(" << cache_name(ni)
         << "[c][j >> 1] >> ((j & 1) * 16));\n";
       emit_leaf_convert(ni);
     } else if (n.kind == RK_LEAF) {
-      o << "      " << stype(R.leaves[n.leaf].dtype) << " (&r" << ni << ")[" << V << "] = cache" << ni << "[c];\n";
+      o << "      " << stype(R.leaves[n.leaf].dtype) << " (&r" << ni << ")[" << V << "] = " << cache_name(ni) << "[c];\n";
       emit_leaf_convert(ni);
     } else {
-      o << "      " << ctype(n.dtype) << " (&f" << ni << ")[" << V << "] = cache" << ni << "[c];\n";
+      o << "      " << ctype(n.dtype) << " (&f" << ni << ")[" << V << "] = " << cache_name(ni) << "[c];\n";
     }
     return;
   }
@@ -866,16 +892,16 @@ void Gen::emit_full_node(int ni, int phase, const std::string& c_expr) {
   }
   if (cached.count(ni) && first_phase[ni] == phase) {
     if (bf16_words(ni))
-      o << "      #pragma unroll\n      for (int jj = 0; jj < " << V / 2 << "; ++jj) cache" << ni << "[c][jj] = rw" << ni
+      o << "      #pragma unroll\n      for (int jj = 0; jj < " << V / 2 << "; ++jj) " << cache_name(ni) << "[c][jj] = rw" << ni
         << "[jj];\n";
     else if (bf16_packed(ni) && n.kind != RK_LEAF)
-      o << "      #pragma unroll\n      for (int jj = 0; jj < " << V / 2 << "; ++jj) cache" << ni
+      o << "      #pragma unroll\n      for (int jj = 0; jj < " << V / 2 << "; ++jj) " << cache_name(ni)
         << "[c][jj] = pack_bf16_exact(f" << ni << "[2 * jj], f" << ni << "[2 * jj + 1]);\n";
     else if (packed_cache(ni))
-      o << "      #pragma unroll\n      for (int j = 0; j < " << V / 2 << "; ++j) cache" << ni << "[c][j] = (u32)r" << ni
+      o << "      #pragma unroll\n      for (int j = 0; j < " << V / 2 << "; ++j) " << cache_name(ni) << "[c][j] = (u32)r" << ni
         << "[2 * j] | ((u32)r" << ni << "[2 * j + 1] << 16);\n";
     else
-      o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) cache" << ni << "[c][j] = "
+      o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) " << cache_name(ni) << "[c][j] = "
         << (n.kind == RK_LEAF ? "r" : "f") << ni << "[j];\n";
   }
 }
@@ -950,9 +976,13 @@ void Gen::emit_red_init(int ni) {
     std::string init;
     if (fvalued(in) || in == DType::F64) init = flt_lit(in == DType::F64 ? DType::F64 : DType::F32, mx ? -INFINITY : INFINITY);
     else init = mx ? int_min(in) : int_max(in);
-    decl(A, "bv" + r, init);
-    decl(aix(), "bi" + r, aix_none());
-    decl("bool", "bn" + r, "false");
+    if (dim.empty()) {
+      o << "  " << A << " bv" << r << " = " << init << "; " << aix() << " bi" << r << " = " << aix_none() << "; bool bn" << r << " = false;\n";
+    } else {
+      decl(A, "bv" + r, init);
+      decl(aix(), "bi" + r, aix_none());
+      decl("bool", "bn" + r, "false");
+    }
     if (chunk_arg(ni)) {
       // the winning chunk: its first element index and its values (bf16 values two to a word)
       o << "  " << aix() << " bc" << r << " = " << aix_none() << "; ";
@@ -981,7 +1011,8 @@ void Gen::emit_red_update(int ni, const std::string& k_expr, const std::string& 
     // reference's NaN-at-index-0 rule (the result is 0) is a flag set by the element k == 0.
     std::string k = "((" + aix() + ")(" + k_expr + "))";
     o << "        { " << ctype(in) << " v_ = " << v << "; if (v_ " << cmp << " " << at("bv" + r, j) << ") { " << at("bv" + r, j)
-      << " = v_; " << at("bi" + r, j) << " = " << k << "; }";
+      << " = v_; " << at("bi" + r, j) << " = " << k << ";"
+      << (tail && mainV >= 2 && fvalued(in) ? " bc" + r + " = " + aix_none() + ";" : "") << " }";
     if (fvalued(in) || in == DType::F64)
       o << " if (" << (col ? "" : j + " == 0 && ") << k << " == 0 && v_ != v_) " << at("bn" + r, j) << " = true;";
     o << " }\n";
@@ -1294,6 +1325,9 @@ std::string Gen::generate(RegionCode* rc) {
   for (auto& l : R.leaves) param(l.slot);
   for (auto& op : R.outputs) param(op.second);
   o << kDevicePrelude;
+  // an output row of that length starts at any element too
+  odd_out = rem != 0;
+  if (odd_out || std::count(leaf_odd.begin(), leaf_odd.end(), true)) o << kDevicePreludeAnyAlign;
   if (Z > 1) {
     mode = PART;
     auto room = [&](size_t width) {
@@ -1366,11 +1400,21 @@ std::string Gen::generate(RegionCode* rc) {
   }
   // ---- line kernel ----
   // caches
-  for (int c : cached) {
-    const RNode& cn = node(c);
-    if (packed_cache(c)) o << "  u32 cache" << c << "[" << NC << "][" << V / 2 << "];\n";
-    else o << "  " << (cn.kind == RK_LEAF ? stype(R.leaves[cn.leaf].dtype) : ctype(cn.dtype)) << " cache" << c << "["
-           << NC << "][" << V << "];\n";
+  auto declare_caches = [&](int chunks) {
+    for (int c : cached) {
+      const RNode& cn = node(c);
+      if (packed_cache(c)) o << "  u32 " << cache_name(c) << "[" << chunks << "][" << V / 2 << "];\n";
+      else o << "  " << (cn.kind == RK_LEAF ? stype(R.leaves[cn.leaf].dtype) : ctype(cn.dtype)) << " " << cache_name(c) << "["
+             << chunks << "][" << V << "];\n";
+    }
+  };
+  declare_caches(NC);
+  if (rem) {
+    tail = true;
+    V = 1;
+    declare_caches(1);
+    tail = false;
+    V = mainV;
   }
   // line-level (level 0) LINE nodes
   for (size_t i = 0; i < R.nodes.size(); ++i)
@@ -1392,7 +1436,7 @@ std::string Gen::generate(RegionCode* rc) {
       kexpr = cexpr + " + j";
     }
     // this thread's chunks: positions first + c * TPL of the line's `total`
-    const uint64_t total = col ? L : (L + V - 1) / V;
+    const uint64_t total = col ? L : L / V;
     const std::string pos = mode == PART ? "((u64)z * " + std::to_string(NC) + "ull + c) * " + std::to_string(TPL) + "ull + lane"
                                          : "(u64)c * " + std::to_string(TPL) + "ull + lane";
     const std::string idt = col ? ix() : "u32", idn = col ? kexpr : "ch";
@@ -1410,10 +1454,13 @@ std::string Gen::generate(RegionCode* rc) {
       o << "  for (int c = 0; c < " << NC << "; ++c) {\n";
       o << "    const " << idt << " " << idn << " = (" << idt << ")c * " << TPL << "u + lane;\n";
       bool guard = (uint64_t)NC * TPL != total;
-      if (guard) o << "    if ((u64)" << idn << " < " << total << "ull) {\n";
+      if (guard && (col || rem)) o << "    if ((u64)" << idn << " < " << total << "ull) {\n";
+      else if (guard) o << "    if ((u64)ch * " << V << "ull < " << L << "ull) {\n";
       else o << "    {\n";
     }
     if (col) emit_bases(false);
+    // one chunk: its values, the reductions they feed and the outputs they are
+    auto emit_chunk = [&](const std::string& cexpr, const std::string& kexpr) {
     for (size_t i = 0; i < R.nodes.size(); ++i)
       if (need[p].count((int)i)) emit_full_node((int)i, p, cexpr);
     for (int r : reds) {
@@ -1442,15 +1489,17 @@ std::string Gen::generate(RegionCode* rc) {
         const bool nts = nt_mode() & 1;
         if (n.dtype == DType::BF16 && V % 2 == 0 && full(op.first)) {
           // every bf16 value is carried bf16-exact in f32: its pattern is the upper half
+          const std::string VT = "VecT<u32, " + std::to_string(V / 2) + ">";
           o << "      { VecT<u32, " << V / 2 << "> w;\n        #pragma unroll\n        for (int jj = 0; jj < " << V / 2
             << "; ++jj) w.v[jj] = pack_bf16_exact(" << val(op.first, "2 * jj") << ", " << val(op.first, "2 * jj + 1")
-            << ");\n        " << (nts ? "vst_nt(" : "*(") << "(VecT<u32, " << V / 2 << ">*)((" << T << "*)" << Pp << " + "
-            << ob.str() << " + (" << ix() << ")(" << cexpr << "))" << (nts ? ", w); }\n" : ") = w; }\n");
+            << ");\n        " << vstore(VT, "(" + T + "*)" + Pp + " + " + ob.str() + " + (" + ix() + ")(" + cexpr + ")", nts, odd_out, dt_width(n.dtype))
+            << "; }\n";
         } else {
+          const std::string VT = "VecT<" + T + ", " + std::to_string(V) + ">";
           o << "      { VecT<" << T << ", " << V << "> w;\n        #pragma unroll\n        for (int j = 0; j < " << V
-            << "; ++j) w.v[j] = " << st(n.dtype, val(op.first, "j")) << ";\n        " << (nts ? "vst_nt(" : "*(")
-            << "(VecT<" << T << ", " << V << ">*)((" << T << "*)" << Pp << " + " << ob.str() << " + (" << ix() << ")("
-            << cexpr << "))" << (nts ? ", w); }\n" : ") = w; }\n");
+            << "; ++j) w.v[j] = " << st(n.dtype, val(op.first, "j")) << ";\n        "
+            << vstore(VT, "(" + T + "*)" + Pp + " + " + ob.str() + " + (" + ix() + ")(" + cexpr + ")", nts, odd_out, dt_width(n.dtype))
+            << "; }\n";
         }
       } else {
         o << "      #pragma unroll\n      for (int j = 0; j < " << V << "; ++j) ((" << T << "*)" << Pp << ")["
@@ -1459,7 +1508,19 @@ std::string Gen::generate(RegionCode* rc) {
       }
       if (col) o << "      }\n";
     }
+    };
+    emit_chunk(cexpr, kexpr);
     o << "    }\n  }\n";
+    if (rem) {
+      tail = true;
+      V = 1;
+      const std::string at = std::to_string(L - rem) + "u + lane";
+      o << "  if (" << (mode == PART ? "z == " + std::to_string(Z - 1) + "u && " : "") << "lane < " << rem << "u) {\n    constexpr int c = 0; (void)c;\n";
+      emit_chunk(at, at + " + j");
+      o << "  }\n";
+      tail = false;
+      V = mainV;
+    }
     for (int r : reds) emit_red_fold(r, p);
     if (mode == PART) {
       for (int r : reds) emit_partials(r);

@@ -147,4 +147,44 @@ KD u16 shx(u16 v, int m) { return (u16)__shfl_xor((i32)v, m, 64); }
 KD bool shx(bool v, int m) { return __shfl_xor((i32)v, m, 64) != 0; }
 )KUPRELUDE";
 
+// The rest of the prelude, for kernels whose rows start at any element.
+inline const char* kDevicePreludeAnyAlign = R"KUPRELUDE(
+// the same accesses (non-temporal or not) at an address aligned to A bytes only: rows of a length
+// that is no multiple of a vector. The hardware takes any alignment.
+template <class V, int A, bool NT> KD V vld_at(const void* p) {
+  typedef ku_u32x4 __attribute__((aligned(4))) x4a4; typedef ku_u32x4 __attribute__((aligned(2))) x4a2; typedef ku_u32x4 __attribute__((aligned(1))) x4a1;
+  typedef ku_u32x2 __attribute__((aligned(4))) x2a4; typedef ku_u32x2 __attribute__((aligned(2))) x2a2; typedef ku_u32x2 __attribute__((aligned(1))) x2a1;
+#define KU_LD(T) (NT ? __builtin_nontemporal_load((const T*)p) : *(const T*)p)
+  if constexpr (sizeof(V) == 16) {
+    if constexpr (A >= 4) return __builtin_bit_cast(V, (ku_u32x4)KU_LD(x4a4));
+    else if constexpr (A == 2) return __builtin_bit_cast(V, (ku_u32x4)KU_LD(x4a2));
+    else return __builtin_bit_cast(V, (ku_u32x4)KU_LD(x4a1));
+  } else if constexpr (sizeof(V) == 8) {
+    if constexpr (A >= 4) return __builtin_bit_cast(V, (ku_u32x2)KU_LD(x2a4));
+    else if constexpr (A == 2) return __builtin_bit_cast(V, (ku_u32x2)KU_LD(x2a2));
+    else return __builtin_bit_cast(V, (ku_u32x2)KU_LD(x2a1));
+  } else {
+    V v;
+    __builtin_memcpy(&v, p, sizeof(V));
+    return v;
+  }
+#undef KU_LD
+}
+template <class V, int A, bool NT> KD void vst_at(void* p, const V& v) {
+  typedef ku_u32x4 __attribute__((aligned(4))) x4a4; typedef ku_u32x4 __attribute__((aligned(2))) x4a2; typedef ku_u32x4 __attribute__((aligned(1))) x4a1;
+  typedef ku_u32x2 __attribute__((aligned(4))) x2a4; typedef ku_u32x2 __attribute__((aligned(2))) x2a2; typedef ku_u32x2 __attribute__((aligned(1))) x2a1;
+#define KU_ST(T, X) { if constexpr (NT) __builtin_nontemporal_store(X, (T*)p); else *(T*)p = X; }
+  if constexpr (sizeof(V) == 16) {
+    const ku_u32x4 x = __builtin_bit_cast(ku_u32x4, v);
+    if constexpr (A >= 4) KU_ST(x4a4, x) else if constexpr (A == 2) KU_ST(x4a2, x) else KU_ST(x4a1, x)
+  } else if constexpr (sizeof(V) == 8) {
+    const ku_u32x2 x = __builtin_bit_cast(ku_u32x2, v);
+    if constexpr (A >= 4) KU_ST(x2a4, x) else if constexpr (A == 2) KU_ST(x2a2, x) else KU_ST(x2a1, x)
+  } else {
+    __builtin_memcpy(p, &v, sizeof(V));
+  }
+#undef KU_ST
+}
+)KUPRELUDE";
+
 }  // namespace ku::hipbk

@@ -357,7 +357,7 @@ attn_mfma_k(AttnArgs a) {
       float rs[2] = {0.f, 0.f};
       // SPLIT_P in f16: probabilities times 2^7 (at most 2^15 with the lazy maximum), so that the
       // remainders of all but the smallest are normal f16 numbers; the row sum carries the factor too
-      const float em = (SPLIT_P && DT == GT_F16 ? 7.f : 0.f) - mc[0];
+      const float em = SPLIT_P && DT == GT_F16 ? 7.f - mc[0] : -mc[0];
       u32x4 kf[3];
       kf[0] = kread(0);
       kf[1] = kread(1);
