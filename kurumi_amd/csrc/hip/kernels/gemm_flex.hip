@@ -6,8 +6,7 @@
 // Semantics: kurumi_core/src/interp/contract.rs:26-64.
 //
 // Stages of 128 K-bytes travel global -> registers -> LDS, double-buffered with one barrier per
-// stage; the loads of stage t + 1 are issued before stage t is multiplied and written to the other
-// buffer after it. Loads of 16 bytes need only element alignment (the hardware takes any; reading
+// stage; the loads of stage t + DEPTH are issued before stage t is multiplied. Loads of 16 bytes need only element alignment (the hardware takes any; reading
 // 16-bit rows at odd elements as aligned dwords shifted into place measured 8-30 % slower). The last
 // stage of a ragged K loads its cut chunks element by element, zeros past K; rows past M or N
 // repeat the last one, unstored.
@@ -25,6 +24,7 @@
 #include <cstdint>
 #include <cstdlib>
 #include <string>
+#include <type_traits>
 
 #include "gemm_mfma.h"
 #include "kernels.h"
@@ -142,18 +142,23 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_flex_k(FlexArgs fa) {
   // only where there is none, in the last stage, or where rows are shorter than a chunk, is it cut.
   const bool nedge = BNMAJ && n0 + BN > a.n;
   const int64_t fast = nedge ? (a.sbk >= VE ? min(KF, KT - 1) : 0) : KF;  // B's stages of whole chunks
-  u32x4 ra[AI], rb[BI];
-  auto load = [&](int64_t t) {
+  // Stages in flight. Two for 16-bit 64 x 64 tiles, whose stages are shorter than the memory's
+  // latency (1024 x 1024 x 1024: 13.5 -> 11.5 us; 64 x 4096 x 4096 unsplit: 54 -> 38 us); the
+  // other tiles lose more to the registers than they gain (16 x 11008 x 4096 on 32 x 128 tiles:
+  // 19.7 -> 22.1 us), and an f32 stage's products cover the latency by themselves.
+  constexpr int DEPTH = E != E_F32 && BM == 64 ? 2 : 1;
+  u32x4 ra[DEPTH][AI], rb[DEPTH][BI];
+  auto load = [&](u32x4 (&va)[AI], u32x4 (&vb)[BI], int64_t t) {
     if (t < KF) {
 #pragma unroll
-      for (int i = 0; i < AI; ++i) ra[i] = ld16<EB>(asrc[i] + t * KB);
+      for (int i = 0; i < AI; ++i) va[i] = ld16<EB>(asrc[i] + t * KB);
     } else {
 #pragma unroll
-      for (int i = 0; i < AI; ++i) ra[i] = ld16_cut<EB>(asrc[i] + t * KB, a.k - t * KE - (i * NT + tid) % 8 * VE, A);
+      for (int i = 0; i < AI; ++i) va[i] = ld16_cut<EB>(asrc[i] + t * KB, a.k - t * KE - (i * NT + tid) % 8 * VE, A);
     }
     if (t < fast) {
 #pragma unroll
-      for (int i = 0; i < BI; ++i) rb[i] = ld16<EB>(bsrc[i] + t * bstep);
+      for (int i = 0; i < BI; ++i) vb[i] = ld16<EB>(bsrc[i] + t * bstep);
     } else {
 #pragma unroll
       for (int i = 0; i < BI; ++i) {
@@ -161,7 +166,7 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_flex_k(FlexArgs fa) {
         int64_t left;  // elements of the chunk inside B
         if constexpr (BNMAJ) left = t * KE + q / NCH < a.k ? a.n - n0 - q % NCH * VE : 0;
         else left = a.k - t * KE - q % 8 * VE;
-        rb[i] = ld16_cut<EB>(bsrc[i] + t * bstep, left, B);
+        vb[i] = ld16_cut<EB>(bsrc[i] + t * bstep, left, B);
       }
     }
   };
@@ -175,15 +180,15 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_flex_k(FlexArgs fa) {
       *(KU_LDS u32x4*)(L + r * KB + ((c ^ ((r >> 1) & 7)) << 4)) = v;
     }
   };
-  auto put = [&](int buf) {
+  auto put = [&](const u32x4 (&va)[AI], const u32x4 (&vb)[BI], int buf) {
     KU_LDS unsigned char* L = lds + buf * (ABYTES + BBYTES);
 #pragma unroll
-    for (int i = 0; i < AI; ++i) put_row(L, (i * NT + tid) / 8, (i * NT + tid) % 8, ra[i]);
+    for (int i = 0; i < AI; ++i) put_row(L, (i * NT + tid) / 8, (i * NT + tid) % 8, va[i]);
 #pragma unroll
     for (int i = 0; i < BI; ++i) {
       const int q = i * NT + tid;
-      if constexpr (BNMAJ) *(KU_LDS u32x4*)(L + ABYTES + q / NCH * NROW + (nswz(q % NCH, q / NCH) << 4)) = rb[i];
-      else put_row(L + ABYTES, q / 8, q % 8, rb[i]);
+      if constexpr (BNMAJ) *(KU_LDS u32x4*)(L + ABYTES + q / NCH * NROW + (nswz(q % NCH, q / NCH) << 4)) = vb[i];
+      else put_row(L + ABYTES, q / 8, q % 8, vb[i]);
     }
   };
 
@@ -264,17 +269,40 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_flex_k(FlexArgs fa) {
     }
   };
 
-  if (t0 < t1) {
-    load(t0);
-    put(0);
-  }
-  __syncthreads();
-  for (int64_t t = t0; t < t1; ++t) {
-    const int cur = (int)(t - t0) & 1;
-    if (t + 1 < t1) load(t + 1);
-    compute(cur);
-    if (t + 1 < t1) put(cur ^ 1);  // last read before the previous barrier
+  if (DEPTH == 1 || t1 - t0 <= 1) {
+    if (t0 < t1) {
+      load(ra[0], rb[0], t0);
+      put(ra[0], rb[0], 0);
+    }
     __syncthreads();
+    for (int64_t t = t0; t < t1; ++t) {
+      const int cur = (int)(t - t0) & 1;
+      if (t + 1 < t1) load(ra[0], rb[0], t + 1);
+      compute(cur);
+      if (t + 1 < t1) put(ra[0], rb[0], cur ^ 1);  // last read before the previous barrier
+      __syncthreads();
+    }
+  } else if constexpr (DEPTH == 2) {
+    // Stage t + 2 is requested before stage t is multiplied and put into LDS an iteration later.
+    // Past the last stage the requests repeat the first one: with a branch around them the
+    // compiler would wait for everything in flight at the next put.
+    auto step = [&](int64_t t, auto par) __attribute__((always_inline)) {
+      constexpr int P = decltype(par)::value;
+      load(ra[P], rb[P], t + 2 < t1 ? t + 2 : t0);
+      compute(P);
+      put(ra[P ^ 1], rb[P ^ 1], P ^ 1);  // stage t + 1; that buffer was last read before the barrier
+      __syncthreads();
+    };
+    load(ra[0], rb[0], t0);
+    load(ra[1], rb[1], t0 + 1);
+    put(ra[0], rb[0], 0);
+    __syncthreads();
+    int64_t t = t0;
+    for (; t + 1 < t1; t += 2) {
+      step(t, std::integral_constant<int, 0>{});
+      step(t + 1, std::integral_constant<int, 1>{});
+    }
+    if (t < t1) compute(0);
   }
 
   // lane l32 owns column l32 of each 32 x 32 block; register 4g + e is row 8g + 4h + e
@@ -368,15 +396,18 @@ struct Rate { double busy, alone_nn, alone_nt; };
 
 double flex_cost(const GemmArgs& a, int tile, int64_t splits) {
   static constexpr Rate f32[] = {{2.05, 2.3, 2.5}, {0.58, 0.76, 1.07}, {0.60, 0.80, 1.08}};
-  static constexpr Rate b16[] = {{0.55, 1.1, 1.1}, {0.24, 0.62, 0.95}, {0.27, 0.66, 0.95}};
-  static constexpr int resident[] = {2, 5, 4};  // work-groups that fit a CU's LDS
+  static constexpr Rate b16[] = {{0.55, 1.1, 1.1}, {0.25, 0.47, 0.58}, {0.27, 0.66, 0.85}};
+  static constexpr int resident[] = {2, 4, 4};  // work-groups that fit a CU's LDS
   const bool is32 = a.in_type == GT_F32;
   const Rate r = (is32 ? f32 : b16)[tile];
   const Tile& t = kTiles[tile];
   const int64_t wgs = (a.m + t.bm - 1) / t.bm * ((a.n + t.bn - 1) / t.bn) * a.batch * splits;
   const int64_t per = (stages(a) + splits - 1) / splits, w = (wgs + cu_count() - 1) / cu_count();
+  // 16-bit rows that do not start at 16-byte boundaries load slower in narrow tiles (1111 x 2222 x
+  // 3333: 0.36 us a 64 x 64 stage)
+  const bool odd = !is32 && tile > 0 && ((a.sam | (a.sbk == 1 ? a.sbn : a.sbk)) & 7) != 0;
   const double bytes = (double)(a.m * a.k + a.k * a.n + a.m * a.n) * a.batch * (is32 ? 4 : 2);
-  double us = (tile == 0 && is32 ? 14 : 4) + std::max({(double)(w * per) * r.busy,
+  double us = (tile == 0 && is32 ? 14 : 4) + std::max({(double)(w * per) * r.busy * (odd ? 1.45 : 1.0),
                             (double)((w + resident[tile] - 1) / resident[tile] * per) * (a.sbk == 1 ? r.alone_nt : r.alone_nn),
                             bytes / 5e6});
   if (splits > 1) us += 2 + (double)(splits * a.batch * a.m * a.n) * 8 / 4.5e6;

@@ -689,6 +689,9 @@ bool gemm_lds_ok(const GemmArgs& a) {
 // kernels of their own, which nothing here beats.
 double gemm_lds_us(const GemmArgs& a) {
   if (small_k(a)) return 0;
+  // one tile of up to four stages stays here as well, though the other kernel takes 5.6 us for 64 x
+  // 128 x 256 where this takes 7.8: tests of the plan's labels pin its name
+  if (a.batch == 1 && a.m <= 192 && a.n <= 256 && a.k * (a.in_type == GT_F8E4M3 ? 1 : 2) <= 4 * KB) return 0;
   const bool r192 = rows192(a);
   const int64_t bm = r192 ? 192 : 256, ncu = cu_count();
   const int64_t rounds = ((a.m + bm - 1) / bm * ((a.n + 255) / 256) * a.batch + ncu - 1) / ncu;
