@@ -41,6 +41,14 @@ std::string gemm_variant(const GemmArgs& a) {
 
 size_t gemm_scratch_bytes(const GemmArgs& a) { return path_of(a) == Path::FLEX ? gemm_flex_scratch_bytes(a) : 0; }
 
+double gemm_estimated_us(const GemmArgs& a) {
+  switch (path_of(a)) {
+    case Path::LDS: return gemm_lds_us(a);
+    case Path::FLEX: return gemm_flex_us(a);
+    default: return 1e9;
+  }
+}
+
 void launch_gemm(const GemmArgs& a, hipStream_t s) {
   if (a.batch * a.m * a.n == 0) return;
   switch (path_of(a)) {

@@ -42,6 +42,8 @@ int cu_count();
 std::string gemm_variant(const GemmArgs& a);
 // scratch that the variant uses (0 for most); `a.a` / `a.b` need the alignment of the operands only
 size_t gemm_scratch_bytes(const GemmArgs& a);
+// estimated microseconds of the variant that will run
+double gemm_estimated_us(const GemmArgs& a);
 void launch_gemm(const GemmArgs& a, hipStream_t s);
 
 struct AttnArgs {
@@ -90,6 +92,12 @@ bool quant_mm_fused_ok(const QuantArgs& a);
 size_t quant_tiled_bytes(int64_t n, int64_t k);
 void launch_quant_tile_weights(const uint8_t* qw, uint8_t* wt, int64_t n, int64_t k, hipStream_t s);
 void launch_quant_mm(const QuantArgs& a, hipStream_t s);
+// dequantisation inside the GEMM (gemm_quant.hip): groups of a multiple of 16, any M and act type;
+// mm_scratch: quant_flex_scratch_bytes() for a split K, unsplit without it
+bool quant_flex_ok(const QuantArgs& a);
+bool quant_flex_better(const QuantArgs& a);
+size_t quant_flex_scratch_bytes(const QuantArgs& a);
+void launch_quant_flex(const QuantArgs& a, hipStream_t s);
 
 // Per-tensor e4m3 activation quantisation (linear_e4m3.hip): sx = max|x| * (1/448) and
 // xq = e4m3(x * (1/sx)) over n contiguous elements, in two kernels (absmax partials, then fold

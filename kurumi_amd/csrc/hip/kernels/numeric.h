@@ -50,6 +50,18 @@ __device__ __forceinline__ float d_round_through(int rt, float v) {
   return v;
 }
 
+// field `raw` of a packed quantised weight, dequantised with scale s / min mn; the product is not
+// fused with the min (the reference rounds q * s, then adds)
+template <int BITS, bool SYM>
+__device__ __forceinline__ float d_dequant(uint32_t raw, float s, float mn) {
+  if constexpr (SYM) {
+    const int v = (int)(raw << (32 - BITS)) >> (32 - BITS);
+    return __fmul_rn((float)v, s);
+  } else {
+    return __fadd_rn(__fmul_rn((float)raw, s), mn);
+  }
+}
+
 // storage element -> accumulation type
 template <int DT, class TI, class TA>
 __device__ __forceinline__ TA load_elem(TI x) {

@@ -1113,12 +1113,21 @@ void Planner::visit_quant(NodeId id) {
   Q.wdq_dtype = at;  // bf16 / f16 act: the MFMA GEMM on rounded weights; f32: the generic GEMM
   Q.out_slot = new_slot(SlotKind::Temp, at, Q.m * Q.n * dt_width(at), id);
   // M <= 8: the fused dequant GEMV; int4 with 9 <= M <= 64 (bf16 / f16 act): the fused dequant
-  // MFMA kernel; otherwise dequantise once into wdq, then the GEMM
+  // MFMA kernel; otherwise a GEMM that dequantises as it stages the weight or, with many rows, one
+  // that follows a dequantisation into wdq
   QuantArgs qa;
   qa.m = (int64_t)Q.m; qa.n = (int64_t)Q.n; qa.k = (int64_t)Q.k; qa.group = (int64_t)Q.group;
   qa.bits = Q.bits; qa.sym = Q.sym; qa.act_type = (int)at;
   qa.mins = Q.sym ? nullptr : reinterpret_cast<const uint16_t*>(16);  // shape check only
-  Q.path = quant_gemv_ok(qa) ? QuantStep::GEMV : (quant_mm_ok(qa) ? QuantStep::MFMA : QuantStep::DEQUANT_GEMM);
+  // what the launch will see of the operands' addresses: buffers are 256-byte aligned
+  qa.act = reinterpret_cast<const char*>(256) + Q.act_off * (int64_t)dt_width(at);
+  qa.qw = reinterpret_cast<const uint8_t*>(256) + Q.qw_off;
+  Q.path = quant_gemv_ok(qa)        ? QuantStep::GEMV
+           : quant_mm_ok(qa)        ? QuantStep::MFMA
+           : quant_flex_better(qa) ? QuantStep::FUSED_GEMM
+                                    : QuantStep::DEQUANT_GEMM;
+  if (Q.path == QuantStep::FUSED_GEMM && quant_flex_scratch_bytes(qa))
+    Q.mm_slot = new_slot(SlotKind::Temp, DType::U8, quant_flex_scratch_bytes(qa), id);
   if (Q.path == QuantStep::DEQUANT_GEMM)
     Q.wdq_slot = new_slot(SlotKind::Temp, Q.wdq_dtype, Q.n * Q.k * dt_width(Q.wdq_dtype), id);
   if (Q.path == QuantStep::MFMA) {
@@ -1827,7 +1836,7 @@ void Plan::compile() {
         Q.ws_slot = scratch_slot(gemm_scratch_bytes(a));
       }
       std::ostringstream o;
-      o << (Q.path == QuantStep::GEMV ? "quant_gemv" : Q.path == QuantStep::MFMA ? "quant_mfma" : "quant_dequant+gemm")
+      o << (Q.path == QuantStep::GEMV ? "quant_gemv" : Q.path == QuantStep::MFMA ? "quant_mfma" : Q.path == QuantStep::FUSED_GEMM ? "quant_dequant+gemm_fused" : "quant_dequant+gemm")
         << " int" << Q.bits << (Q.sym ? "s" : "a") << " g"
         << Q.group << " m" << Q.m << " n" << Q.n << " k" << Q.k;
       s.label = o.str();
@@ -1980,6 +1989,9 @@ void Plan::launch_step(const Step& s) {
         a.qw_tiled = true;
       }
       launch_quant_mm(a, st);
+    } else if (Q.path == QuantStep::FUSED_GEMM) {
+      if (Q.mm_slot >= 0) a.mm_scratch = slot_ptr(slots_, Q.mm_slot);
+      launch_quant_flex(a, st);
     } else {
       a.wdq = slot_ptr(slots_, Q.wdq_slot);
       launch_quant_dequant(a, st);

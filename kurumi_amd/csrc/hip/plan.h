@@ -119,11 +119,12 @@ struct GemmStep {
 };
 
 // Weight-only quantized matmul: a fused dequant GEMV (M <= 8), the fused dequant MFMA kernel
-// (int4, 9 <= M <= 64), else a dequantize pass into `wdq_slot` followed by a GEMM of act x wdq^T.
+// (int4, 9 <= M <= 64), a GEMM that dequantises as it stages the weight, or a dequantize pass into
+// `wdq_slot` followed by a GEMM of act x wdq^T.
 // `tile_const`: the MFMA path's fused kernel reads a constant weight from its lane-ordered copy
 // (`qw_tiled`, held by the constant's cache entry).
 struct QuantStep {
-  enum Path { GEMV, MFMA, DEQUANT_GEMM };
+  enum Path { GEMV, MFMA, FUSED_GEMM, DEQUANT_GEMM };
   Path path = GEMV;
   int act_slot = -1, qw_slot = -1, sc_slot = -1, mn_slot = -1, out_slot = -1, wdq_slot = -1, mm_slot = -1;
   int64_t act_off = 0, qw_off = 0, sc_off = 0, mn_off = 0;  // elements
