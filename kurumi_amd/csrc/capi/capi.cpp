@@ -682,7 +682,7 @@ int32_t ku_hip_linear_e4m3(const KuBackend* b, const void* x, uint32_t x_dtype, 
     a.k = (int64_t)k;
     auto& ctx = b->b->ctx();
     ctx.make_current();
-    const size_t need = ku::hipbk::linear_e4m3_scratch_bytes(a.m, a.k);
+    const size_t need = ku::hipbk::linear_e4m3_scratch_bytes(a.m, a.n, a.k);
     void* ws = b->b->workspace(need);
     try {
       ku::hipbk::linear_e4m3(a, ws, need, stream ? static_cast<hipStream_t>(stream) : ctx.stream());

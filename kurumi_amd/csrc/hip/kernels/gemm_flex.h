@@ -55,7 +55,8 @@ template <int EB>
 __device__ __forceinline__ u32x4 ld16(const unsigned char* p) {
   typedef u32x4 __attribute__((aligned(2))) u32x4_2;
   typedef u32x4 __attribute__((aligned(4))) u32x4_4;
-  if constexpr (EB == 4) return *reinterpret_cast<const u32x4_4*>(p);
+  if constexpr (EB == 1) return *reinterpret_cast<const u32x4*>(p);  // e4m3 rows are 16-byte aligned
+  else if constexpr (EB == 4) return *reinterpret_cast<const u32x4_4*>(p);
   else return *reinterpret_cast<const u32x4_2*>(p);
 }
 // The first `n` elements of a chunk, zeros after them (n <= 0: all zeros). Every load is made, at
@@ -64,6 +65,7 @@ __device__ __forceinline__ u32x4 ld16(const unsigned char* p) {
 template <int EB>
 __device__ __forceinline__ u32x4 ld16_cut(const unsigned char* p, int64_t n, const unsigned char* safe) {
   constexpr int VE = 16 / EB;
+  if constexpr (EB == 1) return n > 0 ? ld16<EB>(p) : u32x4{0, 0, 0, 0};  // K a multiple of 128: never cut
   const unsigned char* q = n > 0 ? p : safe;
   const int last = n > 0 ? (int)(n < VE ? n : VE) - 1 : 0;
   u32x4 v = {0, 0, 0, 0};
@@ -101,14 +103,14 @@ __device__ __forceinline__ void store_any(void* c, int64_t i, int out_type, floa
 template <int E, bool BNMAJ, int BM, int BN, int WM, int WN, int QB = 0, bool SYM = false>
 __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_flex_k(FlexArgs fa) {
   constexpr int NT = WM * WN * 64;
-  constexpr int EB = E == E_F32 ? 4 : 2;
+  constexpr int EB = E == E_F32 ? 4 : E == E_FP8 ? 1 : 2;
   constexpr int KE = KB / EB, VE = 16 / EB;     // K elements per stage, elements per 16-byte chunk
   constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
   constexpr int ABYTES = BM * KB, BBYTES = BN * KB;
   constexpr int AI = ABYTES / 16 / NT, BI = BBYTES / 16 / NT;  // chunks per thread and stage
   constexpr int NROW = BN * EB, NCH = NROW / 16;               // n-major B: bytes and chunks per k-row
   static_assert(AI * NT * 16 == ABYTES && BI * NT * 16 == BBYTES, "stage / thread mismatch");
-  static_assert(FM >= 1 && FN >= 1 && NCH >= 8 && !(QB && BNMAJ), "tile");
+  static_assert(FM >= 1 && FN >= 1 && (NCH >= 8 || !BNMAJ) && !(QB && BNMAJ) && !(E == E_FP8 && (BNMAJ || QB)), "tile");
   constexpr int UPR = KE / 16, UI = (BN * UPR + NT - 1) / NT, QW = QB / 2 > 0 ? QB / 2 : 1;  // units per row and thread, words
   __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[2 * (ABYTES + BBYTES)];
   KU_LDS unsigned char* lds = (KU_LDS unsigned char*)lds_raw;
@@ -304,6 +306,23 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_flex_k(FlexArgs fa) {
             for (int j = 0; j < FN; ++j)
               acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(af[i][e]), __uint_as_float(bf[j][e]),
                                                                acc[i][j], 0, 0, 0);
+      }
+    } else if constexpr (E == E_FP8) {
+      // 64 k per MFMA: half-wave h takes 32 consecutive ones, two chunks
+#pragma unroll
+      for (int s = 0; s < KE / 64; ++s) {
+        u32x4 af[FM][2], bf[FN][2];
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+#pragma unroll
+          for (int i = 0; i < FM; ++i) af[i][v] = row16(LA, wm * TM + i * 32 + l32, 4 * s + 2 * h + v);
+#pragma unroll
+          for (int j = 0; j < FN; ++j) bf[j][v] = row16(LB, wn * TN + j * 32 + l32, 4 * s + 2 * h + v);
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) Op<E>::run(acc[i][j], af[i], bf[j]);
       }
     } else {
 #pragma unroll

@@ -59,14 +59,16 @@ void launch_flex(const FlexArgs& f, int tile, hipStream_t s) {
   }
 }
 
-int64_t stages(const GemmArgs& a) { return (a.k * (a.in_type == GT_F32 ? 4 : 2) + KB - 1) / KB; }
+int64_t width(const GemmArgs& a) { return a.in_type == GT_F32 ? 4 : a.in_type == GT_F8E4M3 ? 1 : 2; }
+int64_t stages(const GemmArgs& a) { return (a.k * width(a) + KB - 1) / KB; }
 
 // Estimated microseconds of a tile and split, from sweeps over 35 products (f32 and bf16, both
 // layouts, 1 to 4096 rows, every tile and split): a stage takes `busy` us of a CU's time when
 // enough work-groups share it and `alone` us of latency when one has it to itself (k-contiguous B
 // reads one 128-byte line per row and stage, from rows often a power of two apart: slower alone);
-// reading the operands takes bytes / 5 TB/s whatever the grid; a split adds the fold's launch and
-// the partial sums' round trip. The choice was within 10 % of the best tile and split measured.
+// reading the operands takes bytes / 5 TB/s, more where few work-groups keep loads in flight; a split
+// adds the fold's launch (nearly 4 us where launches are what bounds the stream) and the partial
+// sums' round trip. The choice was within 10 % of the best tile and split measured.
 struct Rate { double busy, alone_nn, alone_nt; };
 
 }  // namespace
@@ -82,12 +84,12 @@ double gemm_flex_cost(const GemmArgs& a, int tile, int64_t splits, double extra,
   const int64_t per = (stages(a) + splits - 1) / splits, w = (wgs + cu_count() - 1) / cu_count();
   // 16-bit rows that do not start at 16-byte boundaries load slower in narrow tiles (1111 x 2222 x
   // 3333: 0.36 us a 64 x 64 stage)
-  const bool odd = !is32 && tile > 0 && ((a.sam | (a.sbk == 1 ? a.sbn : a.sbk)) & 7) != 0;
-  const double bytes = (double)(a.m * a.k + a.m * a.n) * a.batch * (is32 ? 4 : 2) + b_bytes;
+  const bool odd = width(a) == 2 && tile > 0 && ((a.sam | (a.sbk == 1 ? a.sbn : a.sbk)) & 7) != 0;
+  const double bytes = (double)(a.m * a.k + a.m * a.n) * a.batch * width(a) + b_bytes;
   double us = (tile == 0 && is32 ? 14 : 4) + std::max({(double)(w * per) * (r.busy * (odd ? 1.45 : 1.0) + extra),
                             (double)((w + resident[tile] - 1) / resident[tile] * per) * (a.sbk == 1 ? r.alone_nt : r.alone_nn),
-                            bytes / 5e6});
-  if (splits > 1) us += 2 + (double)(splits * a.batch * a.m * a.n) * 8 / 4.5e6;
+                            bytes / 5e6 * (1 + 0.3 * cu_count() / wgs)});
+  if (splits > 1) us += 4 + (double)(splits * a.batch * a.m * a.n) * 8 / 4.5e6;
   return us;
 }
 
@@ -101,7 +103,12 @@ FlexPlan flex_plan(const GemmArgs& a) {
   for (int i = 0; i < 3; ++i) {
     if (i < 2 && kTiles[i].bm >= 2 * a.m) continue;  // more than half of the tile's rows past M
     for (int64_t s = 1; s <= 64 && (s == 1 || kt / s >= 2); s *= 2) {
-      const double us = gemm_flex_cost(a, i, s, 0, (double)(a.k * a.n) * a.batch * (a.in_type == GT_F32 ? 4 : 2));
+      // e4m3: the partial sums fit beside the quantised activation in the static scratch of the entry
+      // point that does not allocate, so that one rule gives the same sums through every entry point
+      if (a.in_type == GT_F8E4M3 && s > 1 &&
+          (uint64_t)(a.batch * (s * a.m * a.n * 4 + a.m * a.k)) > kLinearE4m3ScratchBytes - 8192)
+        break;
+      const double us = gemm_flex_cost(a, i, s, 0, (double)(a.k * a.n) * a.batch * width(a));
       if (us < best.us) best = {i, s, us};
     }
   }
@@ -112,7 +119,13 @@ FlexPlan flex_plan(const GemmArgs& a) {
 
 bool gemm_flex_ok(const GemmArgs& a) {
   if (const char* e = std::getenv("KURUMI_HIP_NO_MFMA"); e && *e && *e != '0') return false;
-  if (!(a.in_type == GT_BF16 || a.in_type == GT_F16 || a.in_type == GT_F32)) return false;
+  if (!(a.in_type == GT_BF16 || a.in_type == GT_F16 || a.in_type == GT_F32 || a.in_type == GT_F8E4M3)) return false;
+  if (a.in_type == GT_F8E4M3) {
+    // whole stages of 16-byte aligned rows, k-contiguous; more than 1024 rows stay with the direct
+    // kernel (its path's tests pin its tiles there, and at a layer's widths they fill the chip)
+    const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    if (a.sbk != 1 || a.k % 128 != 0 || ((a.sam | a.sbn | a.sab | a.sbb) & 15) || !al(a.a) || !al(a.b) || a.m > 1024) return false;
+  }
   if (!(a.out_type == GT_BF16 || a.out_type == GT_F16 || a.out_type == GT_F32)) return false;
   if (a.k <= 0 || a.m <= 0 || a.n <= 0 || a.sak != 1 || !(a.sbk == 1 || a.sbn == 1)) return false;
   return a.batch <= 65535 && (a.m + 31) / 32 * ((a.n + 63) / 64) < ((int64_t)1 << 24);
@@ -128,7 +141,7 @@ size_t gemm_flex_scratch_bytes(const GemmArgs& a) {
 
 std::string gemm_flex_name(const GemmArgs& a) {
   const FlexPlan p = flex_plan(a);
-  std::string n = a.in_type == GT_F32 ? "gemm_mfma_f32" : a.in_type == GT_F16 ? "gemm_mfma_f16" : "gemm_mfma_bf16";
+  std::string n = a.in_type == GT_F8E4M3 ? "gemm_mfma_e4m3" : a.in_type == GT_F32 ? "gemm_mfma_f32" : a.in_type == GT_F16 ? "gemm_mfma_f16" : "gemm_mfma_bf16";
   n += a.sbk == 1 ? "_nt_" : "_nn_";
   n += std::to_string(kTiles[p.tile].bm) + "x" + std::to_string(kTiles[p.tile].bn) + "_flex";
   if (p.splits > 1) n += "_split" + std::to_string(p.splits);
@@ -144,7 +157,8 @@ void launch_gemm_flex_as(const GemmArgs& a, int tile, int64_t splits, hipStream_
   f.per = (int)((kt + splits - 1) / splits);
   f.splits = (int)splits;
   const bool nt = a.sbk == 1;
-  if (a.in_type == GT_F32) nt ? launch_flex<E_F32, false>(f, tile, s) : launch_flex<E_F32, true>(f, tile, s);
+  if (a.in_type == GT_F8E4M3) launch_flex<E_FP8, false>(f, tile, s);
+  else if (a.in_type == GT_F32) nt ? launch_flex<E_F32, false>(f, tile, s) : launch_flex<E_F32, true>(f, tile, s);
   else if (a.in_type == GT_F16) nt ? launch_flex<E_F16, false>(f, tile, s) : launch_flex<E_F16, true>(f, tile, s);
   else nt ? launch_flex<E_BF16, false>(f, tile, s) : launch_flex<E_BF16, true>(f, tile, s);
   if (splits > 1) launch_gemm_fold(&f, s);

@@ -125,8 +125,10 @@ struct LinearE4m3Args {
   int y_type = GT_BF16;
   int64_t m = 0, n = 0, k = 0;
 };
-// bytes of scratch one call needs: absmax partials, sx and the quantised activation (M*K)
+// bytes of scratch one call needs: absmax partials, sx and the quantised activation (M*K); with n,
+// the GEMM's own scratch too (without room for it K is not split)
 size_t linear_e4m3_scratch_bytes(int64_t m, int64_t k);
+size_t linear_e4m3_scratch_bytes(int64_t m, int64_t n, int64_t k);
 void linear_e4m3(const LinearE4m3Args& a, void* scratch, size_t scratch_bytes, hipStream_t s);
 // The same with scratch in a static device array of kLinearE4m3ScratchBytes per GPU (no
 // allocation): m * k <= kLinearE4m3ScratchBytes - 4352. init_ looks the array up on the current GPU.

@@ -21,6 +21,7 @@
 // needs clearing), so calls that overlap on one GPU race.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 #include <stdexcept>
@@ -230,7 +231,17 @@ void check_linear(const LinearE4m3Args& a) {
   if (!al(a.x) || !al(a.wq) || !al(a.y)) throw std::runtime_error("x, wq and y must be 16-byte aligned");
 }
 
-void run_linear(const LinearE4m3Args& a, uint8_t* xq, float* partials, float* sx, hipStream_t s) {
+GemmArgs linear_gemm(int64_t m, int64_t n, int64_t k) {
+  GemmArgs g;
+  g.sam = k; g.sak = 1; g.sab = 0;
+  g.sbn = k; g.sbk = 1; g.sbb = 0;  // B[k][n] = wq[n][k]: the NT layout
+  g.batch = 1; g.m = m; g.n = n; g.k = k;
+  g.in_type = GT_F8E4M3;
+  return g;
+}
+
+// `ws`: what is left of the scratch, for a split K
+void run_linear(const LinearE4m3Args& a, uint8_t* xq, float* partials, float* sx, void* ws, size_t ws_bytes, hipStream_t s) {
   ActQArgs q;
   q.x = a.x;
   q.x_type = a.x_type;
@@ -239,14 +250,12 @@ void run_linear(const LinearE4m3Args& a, uint8_t* xq, float* partials, float* sx
   q.partials = partials;
   q.sx = sx;
   launch_actq(q, s);
-  GemmArgs g;
+  GemmArgs g = linear_gemm(a.m, a.n, a.k);
   g.a = xq;
   g.b = a.wq;
   g.c = a.y;
-  g.sam = a.k; g.sak = 1; g.sab = 0;
-  g.sbn = a.k; g.sbk = 1; g.sbb = 0;  // B[k][n] = wq[n][k]: the NT layout
-  g.batch = 1; g.m = a.m; g.n = a.n; g.k = a.k;
-  g.in_type = GT_F8E4M3;
+  g.ws = ws;
+  g.ws_bytes = ws_bytes;
   g.out_type = a.y_type;
   g.alpha = sx;
   g.col_scale = a.sw;
@@ -290,13 +299,21 @@ uint8_t* scratch_on_current_device() {
 
 size_t linear_e4m3_scratch_bytes(int64_t m, int64_t k) { return kXqOff + (size_t)(m * k); }
 
+// a split K's partial sums follow xq, 256-byte aligned
+static size_t partial_sums_off(int64_t m, int64_t k) { return (linear_e4m3_scratch_bytes(m, k) + 255) / 256 * 256; }
+
+size_t linear_e4m3_scratch_bytes(int64_t m, int64_t n, int64_t k) {
+  return partial_sums_off(m, k) + gemm_scratch_bytes(linear_gemm(m, n, k));
+}
+
 void linear_e4m3(const LinearE4m3Args& a, void* scratch_buf, size_t scratch_bytes, hipStream_t s) {
   check_linear(a);
   if (!scratch_buf || scratch_bytes < linear_e4m3_scratch_bytes(a.m, a.k))
     throw std::runtime_error("scratch buffer too small");
   uint8_t* base = static_cast<uint8_t*>(scratch_buf);
+  const size_t used = std::min(partial_sums_off(a.m, a.k), scratch_bytes);
   run_linear(a, base + kXqOff, reinterpret_cast<float*>(base + kPartialsOff), reinterpret_cast<float*>(base + kSxOff),
-             s);
+             base + used, scratch_bytes - used, s);
 }
 
 void linear_e4m3_noalloc(const LinearE4m3Args& a, hipStream_t s) {
@@ -306,8 +323,9 @@ void linear_e4m3_noalloc(const LinearE4m3Args& a, hipStream_t s) {
                              std::to_string(kLinearE4m3ScratchBytes - kXqOff) +
                              " bytes the static scratch holds for the quantised activation");
   uint8_t* base = scratch_on_current_device();
+  const size_t used = std::min(partial_sums_off(a.m, a.k), kLinearE4m3ScratchBytes);
   run_linear(a, base + kXqOff, reinterpret_cast<float*>(base + kPartialsOff), reinterpret_cast<float*>(base + kSxOff),
-             s);
+             base + used, kLinearE4m3ScratchBytes - used, s);
 }
 
 void init_linear_e4m3_noalloc() { (void)scratch_on_current_device(); }

@@ -1,4 +1,4 @@
-"""The register-staged MFMA GEMM (f32 operands, 16-bit operands of any alignment, split K) against
+"""The register-staged MFMA GEMM (f32 operands, 16-bit operands of any alignment, e4m3, split K) against
 the oracle, bit for bit: operands are multiples of 1/16 in [-1, 1], so every partial sum of up to
 2^16 products is a multiple of 1/256 below 2^16 and exact in f32 in any order."""
 import numpy as np
@@ -82,3 +82,24 @@ def test_f32_products_keep_infinities_nans_and_denormals(hip, m, n, k):
     want[0], want[1], want[1, n - 1] = np.inf, np.float32(1e-41), np.float32(1e-41) * 2
     want[:, 1] = np.nan
     np.testing.assert_array_equal(got, want)
+
+
+# few tiles, cut by M and N; one stage and many; split and unsplit; the last of the rows that take it
+@pytest.mark.parametrize("m,n,k", [(1, 64, 128), (33, 70, 256), (16, 512, 4096), (130, 100, 640), (300, 520, 384), (1024, 65, 128), (7, 3000, 2048)])
+def test_e4m3_products_of_few_tiles_match_oracle(hip, m, n, k):
+    """The e4m3 linear's product (operands multiples of 1/16, exact in e4m3, unit scales) in f32."""
+    print(f"e4m3 {m}x{n}x{k}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    codes = np.array([0x00, 0x18, 0x20, 0x28, 0x30, 0x38, 0x98, 0xa0, 0xa8, 0xb0, 0xb8], np.uint8)  # 0, +-2^-4 .. +-1
+    g = K.Graph()
+    a, b = g.input([m, k], DType.F8E4M3), g.input([n, k], DType.F8E4M3)
+    sx, sw = g.input([1], DType.F32), g.input([n], DType.F32)
+    d = g.dot_general(g.cast(a, DType.F32), g.cast(b, DType.F32), [1], [1])
+    d = g.mul(d, g.expand(g.reshape(sx, [1, 1]), [m, n]))
+    y = g.cast(g.mul(d, g.expand(g.reshape(sw, [1, n]), [m, n])), DType.BF16)
+    feeds = {a: Tensor(DType.F8E4M3, (m, k), rng.choice(codes, (m, k)).tobytes()), b: Tensor(DType.F8E4M3, (n, k), rng.choice(codes, (n, k)).tobytes()),
+             sx: tensor([0.5], DType.F32), sw: tensor(2.0 ** rng.integers(-2, 3, n), DType.F32)}
+    plan = hip.plan(g, [y], feeds)
+    assert plan.steps()[-1].startswith("gemm_mfma_e4m3"), plan.steps()
+    plan.launch()
+    np.testing.assert_array_equal(plan.output(0).numpy(), interpret(g, [y], feeds)[0].numpy())
