@@ -590,17 +590,31 @@ void launch_tile(const GemmArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((gemm_lds_k<E, BNMAJ, OT, BM, BN, WM, WN, false, OCC>), grid, dim3(WM * WN * 64), 0, s, a);
 }
 
-// One work-group per CU at a time (the stages fill the LDS), so the tiles run in rounds of
-// cu_count(). 192-row tiles win when they need no more rounds than 256-row ones by enough to
-// outweigh their ~10 % lower efficiency (a 96 x 64 wave tile reads more LDS per MFMA): measured
-// on the e4m3 [2048, 4096] x [11008, 4096]^T linear, 344 tiles of 256 x 256 (2 rounds, the second
-// a third full) 101 us vs 473 tiles of 192 x 256 (2 full rounds) 90 us; the bf16
-// [4096, 4096] x [4096, 11008] GEMM keeps 256 rows (359 vs 379 us).
-bool rows192(const GemmArgs& a) {
-  const int64_t ncu = cu_count(), tn = (a.n + 255) / 256;
-  const int64_t r256 = ((a.m + 255) / 256 * tn * a.batch + ncu - 1) / ncu;
-  const int64_t r192 = ((a.m + 191) / 192 * tn * a.batch + ncu - 1) / ncu;
-  return (double)r192 * 192 * 1.1 < (double)r256 * 256;
+// Tile shapes. One 256- or 192-row work-group fits a CU at a time (its stages fill the LDS), so such
+// tiles run in rounds of cu_count(); two 128 x 128 ones share a CU. Estimated microseconds per
+// stage, from bf16 products of 16 to 4096 rows: 1.2 per round of 256-row tiles, 1.0 of 192-row ones
+// (a 96 x 64 wave tile reads more LDS per MFMA), 0.47 per 128 x 128 tile of a CU and at least 0.8.
+//   e4m3 [2048, 4096] x [11008, 4096]^T: 344 tiles of 256 x 256 take two rounds, the second a third
+//     full, 101 us; 473 tiles of 192 x 256 two full rounds, 90 us
+//   bf16 [4096, 4096] x [4096, 11008]: 256 rows 359 us, 192 rows 379 us
+//   bf16 1500 x 4096 x 4096: 256 rows 87 us, 128 x 128 62 us; 600 x 11008 x 4096: 192 rows 66 us,
+//     128 x 128 58 us; 2048 x 11008 x 4096: 256 rows 160 us, 128 x 128 176 us
+enum LdsTile : int { T256 = 0, T192 = 1, T128 = 2 };
+
+double tile_us(const GemmArgs& a, LdsTile t) {
+  static constexpr int bm[] = {256, 192, 128}, bn[] = {256, 256, 128};
+  static constexpr double stage[] = {1.2, 1.0, 0.47};
+  const int64_t ncu = cu_count(), kt = a.k * (a.in_type == GT_F8E4M3 ? 1 : 2) / KB;
+  const int64_t per_cu = ((a.m + bm[t] - 1) / bm[t] * ((a.n + bn[t] - 1) / bn[t]) * a.batch + ncu - 1) / ncu;
+  return 4 + (double)kt * std::max((double)per_cu * stage[t], t == T128 ? 0.8 : 0.0);
+}
+
+LdsTile lds_tile(const GemmArgs& a) {
+  const LdsTile big = 0.99 * (tile_us(a, T192) - 4) < tile_us(a, T256) - 4 ? T192 : T256;
+  // e4m3 keeps the big tiles, as does one tile of up to four stages (both named in the plan's labels
+  // that tests pin; 64 x 128 x 256 takes 7.8 us on the big tile)
+  if (a.in_type == GT_F8E4M3 || (a.batch == 1 && a.m <= 192 && a.n <= 256 && a.k * 2 <= 4 * KB)) return big;
+  return tile_us(a, T128) < tile_us(a, big) ? T128 : big;
 }
 
 // small K (one or two stages): 128 x 128 tiles of 4 waves, two work-groups per CU, so one
@@ -637,7 +651,8 @@ void launch_cfg(const GemmArgs& a, hipStream_t s) {
     if (smallk_persistent(a)) return launch_smallk<E, BNMAJ, OT>(a, s);
   }
   if (small_k(a)) launch_tile<E, BNMAJ, OT, 128, 128, 2, 2, 2>(a, s);
-  else if (rows192(a)) launch_tile<E, BNMAJ, OT, 192, 256, 2, 4>(a, s);
+  else if (lds_tile(a) == T128) launch_tile<E, BNMAJ, OT, 128, 128, 2, 2, 2>(a, s);
+  else if (lds_tile(a) == T192) launch_tile<E, BNMAJ, OT, 192, 256, 2, 4>(a, s);
   else launch_tile<E, BNMAJ, OT, 256, 256, 2, 4>(a, s);
 }
 
@@ -684,25 +699,20 @@ bool gemm_lds_ok(const GemmArgs& a) {
   return a.batch <= 65535;
 }
 
-// Estimated microseconds: rounds of one tile per CU, 1.2 us per stage of a 256-row tile (1.0 of a
-// 192-row one), measured on bf16 products from 16 to 2048 rows. Products of one or two stages have
-// kernels of their own, which nothing here beats.
+// Estimated microseconds. Products of one or two stages have kernels of their own, which nothing
+// else beats.
 double gemm_lds_us(const GemmArgs& a) {
   if (small_k(a)) return 0;
   // one tile of up to four stages stays here as well, though the other kernel takes 5.6 us for 64 x
   // 128 x 256 where this takes 7.8: tests of the plan's labels pin its name
   if (a.batch == 1 && a.m <= 192 && a.n <= 256 && a.k * (a.in_type == GT_F8E4M3 ? 1 : 2) <= 4 * KB) return 0;
-  const bool r192 = rows192(a);
-  const int64_t bm = r192 ? 192 : 256, ncu = cu_count();
-  const int64_t rounds = ((a.m + bm - 1) / bm * ((a.n + 255) / 256) * a.batch + ncu - 1) / ncu;
-  const int64_t kt = a.k * (a.in_type == GT_F8E4M3 ? 1 : 2) / KB;
-  return 4 + (double)(rounds * kt) * (r192 ? 1.0 : 1.2);
+  return tile_us(a, lds_tile(a));
 }
 
 std::string gemm_lds_name(const GemmArgs& a) {
   std::string n = a.in_type == GT_F8E4M3 ? "gemm_mfma_e4m3" : a.in_type == GT_F16 ? "gemm_mfma_f16" : "gemm_mfma_bf16";
   n += a.sbk == 1 ? "_nt" : "_nn";
-  n += smallk_persistent(a) ? "_128x128_persistent" : small_k(a) ? "_128x128" : rows192(a) ? "_192x256" : "_256x256";
+  n += smallk_persistent(a) ? "_128x128_persistent" : small_k(a) || lds_tile(a) == T128 ? "_128x128" : lds_tile(a) == T192 ? "_192x256" : "_256x256";
   if (!spans_fit(a)) n += "_a64";
   return n;
 }

@@ -25,7 +25,7 @@ def sixteenths(rng, shape):
 # tiles cut by M, N and K, one element, one column, rows of odd length, whole tiles, long K on few
 # tiles (split), more rows than one tile of each height, aligned products of few tiles
 SIZES = [(1, 1, 1), (2, 3, 5), (33, 1, 70), (1, 130, 129), (31, 65, 127), (64, 64, 64), (130, 129, 33), (7, 128, 2496),
-         (257, 300, 95), (5, 7, 9001), (200, 120, 1111), (16, 512, 1024), (300, 264, 2048)]
+         (257, 300, 95), (1030, 1400, 256), (5, 7, 9001), (200, 120, 1111), (16, 512, 1024), (300, 264, 2048)]
 
 
 @pytest.mark.parametrize("m,n,k", SIZES)
