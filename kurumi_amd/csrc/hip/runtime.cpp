@@ -220,6 +220,7 @@ Context::~Context() {
       if (stage_ev_[i]) (void)hipEventDestroy(stage_ev_[i]);
       if (stage_[i]) (void)hipHostFree(stage_[i]);
     }
+    if (small_) (void)hipHostFree(small_);
     (void)hipStreamDestroy(stream_);
   }
 }
@@ -228,6 +229,10 @@ namespace {
 constexpr size_t kStageChunk = size_t(32) << 20;
 // Below this a pageable copy's fixed cost is lower than the staging loop's.
 constexpr size_t kStageMin = size_t(4) << 20;
+// Up to here a download lands in pinned memory and is copied on: the runtime's own path to pageable
+// memory takes 20.8 us for 1.3 KB and 27.2 us for 16 KB, this one 11.5 and 12.1 us (an empty kernel
+// and a wait: 10.8 us). At 100 KB the two are equal.
+constexpr size_t kSmall = size_t(64) << 10;
 }  // namespace
 
 bool Context::ensure_stage() {
@@ -267,6 +272,22 @@ void Context::upload(void* dev, const void* host, size_t n) {
 
 void Context::download(void* host, const void* dev, size_t n) {
   if (!n) return;
+  // A second thread that finds the buffer taken copies straight to its own memory instead of waiting.
+  std::unique_lock<std::mutex> own(small_mu_, std::defer_lock);
+  if (n <= kSmall && own.try_lock()) {
+    if (!small_ && !small_failed_ && hipHostMalloc(&small_, kSmall, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      small_ = nullptr;
+      small_failed_ = true;
+    }
+    if (small_) {
+      KU_HIP(hipMemcpyAsync(small_, dev, n, hipMemcpyDeviceToHost, stream_));
+      sync();
+      std::memcpy(host, small_, n);
+      return;
+    }
+    own.unlock();
+  }
   if (n < kStageMin || !ensure_stage()) {
     KU_HIP(hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, stream_));
     sync();

@@ -123,6 +123,9 @@ class Context {
   hipEvent_t stage_ev_[2] = {nullptr, nullptr};
   bool stage_recorded_[2] = {false, false};
   bool stage_failed_ = false;
+  std::mutex small_mu_;    // plans of several threads download through one Context
+  void* small_ = nullptr;  // pinned landing place of small downloads
+  bool small_failed_ = false;
 };
 
 }  // namespace ku::hipbk
