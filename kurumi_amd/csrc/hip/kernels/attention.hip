@@ -21,7 +21,8 @@ bool attention_f32_ok(const AttnArgs& a);
 
 namespace {
 
-// Reference-grade fallback: one thread per query row, online softmax in registers.
+// Sequences of a few positions and unaligned buffers: one thread per query row, online softmax in
+// registers. A serial chain over the keys, so its time grows with them.
 template <int D, int DT, class T>
 __global__ void __launch_bounds__(64) attn_rowwise_k(AttnArgs a) {
   const int64_t head = blockIdx.y;
@@ -67,6 +68,16 @@ void launch_rowwise(const AttnArgs& a, hipStream_t s) {
     default: throw std::runtime_error("kurumi_hip attention: unsupported dtype");
   }
 }
+// The tiled kernels' time is that of their one tile of 32 queries or more however few it holds, a
+// query's chain costs 0.7 to 2.5 us a key. 25 heads, this kernel against the tiled one (us):
+//   f32, d 32:   1 position 3.7 / 5.0, 4 positions 4.3 / 5.0, 5 positions 5.0 / 4.8
+//   f32, d 64:   1: 3.7 / 6.6, 5: 6.1 / 6.3, 8: 8.6 / 6.6
+//   f32, d 128:  1: 4.9 / 11.4, 3: 9.9 / 10.7, 4: 12.4 / 11.5
+//   f16, d 32:   1: 3.6 / 5.2, 4: 4.9 / 5.2, 5: 5.8 / 5.2
+// 16-bit heads of 64 and 128 stay with the tiled kernel at every length.
+bool few_positions(const AttnArgs& a) {
+  return (a.dtype == GT_F32 || a.d == 32) && a.s <= (a.d == 128 ? 3 : a.d == 64 ? 5 : 4) && a.bh <= 65535;
+}
 
 }  // namespace
 
@@ -77,6 +88,7 @@ bool attn_supported(const AttnArgs& a) {
 }
 
 const char* attn_variant(const AttnArgs& a) {
+  if (few_positions(a)) return "attn_rowwise";
   if (attention_mfma_ok(a)) return "attn_mfma";
   if (attention_f32_ok(a)) return "attn_mfma_f32";
   return "attn_rowwise";
@@ -84,11 +96,12 @@ const char* attn_variant(const AttnArgs& a) {
 
 void launch_attention(const AttnArgs& a, hipStream_t s) {
   if (!attn_supported(a)) throw std::runtime_error("kurumi_hip attention: unsupported shape");
-  if (attention_mfma_ok(a)) {
+  const bool few = few_positions(a);
+  if (!few && attention_mfma_ok(a)) {
     launch_attention_mfma(a, s);
     return;
   }
-  if (attention_f32_ok(a)) {
+  if (!few && attention_f32_ok(a)) {
     launch_attention_f32(a, s);
     return;
   }

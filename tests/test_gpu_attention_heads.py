@@ -39,9 +39,10 @@ def run(hip, dt, arrays, causal, label):
     return to_f32(plan.output(0))
 
 
-# one query; a tile less one and plus one; keys for one, some and all of a group's four waves; a
-# last partial block in each
-SHAPES = [(1, 1, 1), (2, 1, 31), (1, 3, 33), (1, 2, 100), (2, 2, 128), (1, 2, 500), (1, 1, 1000)]
+# one query; on both sides of the few positions that take the one-query-per-thread kernel (to 4
+# with heads of 32, 5 with 64, 3 with 128); a tile less one and plus one; keys for one, some and all of a group's four
+# waves; a last partial block in each
+SHAPES = [(1, 1, 1), (1, 3, 2), (2, 5, 3), (1, 5, 4), (1, 5, 5), (1, 2, 6), (2, 1, 31), (1, 3, 33), (1, 2, 100), (2, 2, 128), (1, 2, 500), (1, 1, 1000)]
 
 
 @pytest.mark.parametrize("b,h,s", SHAPES)
@@ -52,7 +53,7 @@ def test_f32_attention_matches_f64(hip, b, h, s, d, causal, std):
     print(f"f32 attention {b}x{h}x{s}x{d} causal={causal} std={std}", flush=True)
     rng = np.random.default_rng(s * 10 + d)
     q, k, v = (rng.standard_normal((b, h, s, d)).astype(np.float32) * np.float32(x) for x in (std, 1.0, 1.0))
-    got = run(hip, DType.F32, [q, k, v], causal, "attn_mfma_f32")
+    got = run(hip, DType.F32, [q, k, v], causal, "attn_rowwise" if s <= {32: 4, 64: 5, 128: 3}[d] else "attn_mfma_f32")
     want = f64_attention(*(x.astype(np.float64) for x in (q, k, v)), causal)
     assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
 
@@ -65,7 +66,7 @@ def test_16_bit_heads_of_32_match_f64(hip, b, h, s, dt, causal):
     rng = np.random.default_rng(s)
     arrays = [rng.standard_normal((b, h, s, 32)).astype(np.float32) for _ in range(3)]
     arrays = [bf16_bits_to_f32(f32_to_bf16_bits(x)) if dt == DType.BF16 else x.astype(np.float16).astype(np.float32) for x in arrays]
-    got = run(hip, dt, arrays, causal, "attn_mfma ")
+    got = run(hip, dt, arrays, causal, "attn_rowwise" if s <= 4 else "attn_mfma ")
     # the scale is a scalar of the operands' type
     scale = np.float32(32 ** -0.5)
     scale = bf16_bits_to_f32(f32_to_bf16_bits(scale)) if dt == DType.BF16 else np.float16(scale)
