@@ -569,8 +569,8 @@ static bool splittable(const Region& R) {
 // coalesce; a work-group's threads along the axis fold through LDS. Before, one thread walked one
 // whole line, so a launch had `lines` threads and each a serial chain of L loads: the f32
 // [16384, 1000] column sum took 2413 us on 4 work-groups and takes 20.5 us (65.5 MB, 3.2 TB/s,
-// both launches) on 1024 work-groups of 64 x 4 threads and 256 slices. Bound by the read, the ramp
-// and drain of two short launches.
+// both launches) on 1024 work-groups of 64 x 4 threads and 256 slices: 11.9 us
+// for the slices, the rate of a large copy, and 8.7 us for the fold of their 1 MB of partial sums.
 void Gen::plan_columns() {
   const uint64_t threads = (uint64_t)1 << 18;  // 16 waves per CU
   const bool split = splittable(R);

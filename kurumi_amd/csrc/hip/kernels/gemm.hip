@@ -1,6 +1,7 @@
 // GEMM dispatch: the direct-to-LDS MFMA kernel (gemm_lds.hip) for the bf16 / f16 / e4m3
-// layouts it covers and fills the chip with, the register-staged MFMA kernel (gemm_flex.hip) for the other 16-bit products
-// and for f32, the generic tiled kernel (gemm_generic.hip) for everything else.
+// layouts it covers and fills the chip with, the register-staged MFMA kernel (gemm_flex.hip) for the
+// other products of these types and for f32, the generic tiled kernel (gemm_generic.hip) for
+// everything else.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -23,7 +24,7 @@ enum class Path { LDS, FLEX, GENERIC };
 Path path_of(const GemmArgs& a) {
   // Where both take the product, the direct-to-LDS kernel wins when its big tiles fill the chip and
   // loses when they do not (bf16, K x N = 4096 x 11008: 16 rows 63 against 20 us, 300 rows with
-  // 2048 x 5504 42 against 25 us; 600 rows 66 against 73 us, 2048 rows 160 against 236 us), so the
+  // 2048 x 5504 42 against 25 us; 600 rows 58 against 73 us, 2048 rows 160 against 236 us), so the
   // two kernels' estimates are compared; within 10 % of each other the direct one is kept.
   const bool flex = gemm_flex_ok(a);
   if (gemm_lds_ok(a)) return flex && 1.1 * gemm_flex_us(a) < gemm_lds_us(a) ? Path::FLEX : Path::LDS;

@@ -6,8 +6,8 @@
 // Semantics: kurumi_core/src/interp/contract.rs:26-64.
 //
 // Stages of 128 K-bytes travel global -> registers -> LDS, double-buffered with one barrier per
-// stage; the loads of stage t + DEPTH are issued before stage t is multiplied. Loads of 16 bytes need only element alignment (the hardware takes any; reading
-// 16-bit rows at odd elements as aligned dwords shifted into place measured 8-30 % slower). The last
+// stage; the loads of stage t + DEPTH are issued before stage t is multiplied. Loads of 16
+// bytes need only element alignment (the hardware takes any; reading 16-bit rows at odd elements as aligned dwords shifted into place measured 8-30 % slower). The last
 // stage of a ragged K loads its cut chunks element by element, zeros past K; rows past M or N
 // repeat the last one, unstored.
 // LDS layouts are those of gemm_lds.hip (128-byte rows with swizzled chunks; n-major B read with

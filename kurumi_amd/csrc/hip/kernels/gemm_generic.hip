@@ -1,9 +1,9 @@
 // Generic batched GEMM for every dtype and stride pattern the contraction lowering can
 // produce: C[b][m][n] = sum_k A[b][m][k] * B[b][k][n]. Low-precision floats accumulate in
 // f32 and round once at the store; f64 accumulates in f64; integers wrap
-// (kurumi_core/src/interp/contract.rs:26-64,101-144). The MFMA kernels (gemm_mfma.hip)
-// take the bf16/f16/fp8 shapes that matter for speed; this one keeps every other case on
-// the device.
+// (kurumi_core/src/interp/contract.rs:26-64,101-144). The MFMA kernels (gemm_lds.hip,
+// gemm_flex.hip) take f32, bf16, f16 and e4m3 with one unit stride an operand; this one keeps every
+// other case on the device.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
