@@ -481,6 +481,7 @@ void Gen::plan_layout() {
   lines = 1;
   for (int d = 0; d < rank; ++d)
     if (d != (flat ? rank - 1 : a)) lines *= R.S[d];
+  if (!flat && lines == 0) return;  // nothing to lay out (generate() emits no work)
   // vector width: 16 bytes of the narrowest streamed type, only along a contiguous last axis
   int minw = 8;
   for (auto& l : R.leaves)
@@ -1314,7 +1315,6 @@ void Gen::emit_fold_kernel(const std::string& entry) {
 
 std::string Gen::generate(RegionCode* rc) {
   plan_layout();
-  schedule();
   std::ostringstream nm;
   // placeholder entry; the final name carries the iteration shape and a hash of the body so
   // that profiles can tell kernels apart (one name per distinct generated kernel)
@@ -1322,6 +1322,13 @@ std::string Gen::generate(RegionCode* rc) {
   for (size_t d = 0; d < R.S.size(); ++d) nm << (d ? "x" : "_") << R.S[d];
   std::string entry = "KU_ENTRY_PLACEHOLDER";
   std::string prefix = nm.str();
+  if (!flat && lines == 0) {  // every output is empty: a kernel of grid 0, which is never launched
+    o << "extern \"C\" __global__ void " << entry << "() {}\n";
+    rc->grid = 0;
+    rc->block = 64;
+    return finish(prefix, rc);
+  }
+  schedule();
   for (auto& l : R.leaves) param(l.slot);
   for (auto& op : R.outputs) param(op.second);
   o << kDevicePrelude;

@@ -328,3 +328,14 @@ def test_fp8_epilogue_matcher_takes_column_scales_only():
     g, _, y = _scaled_fp8_dot(256, 256, 128, per_row=True)
     st = steps(g.codegen([y], compile=True))
     assert not any(s.startswith("gemm_mfma_e4m3") for s in st), st
+
+
+@pytest.mark.parametrize("kind", ["sum", "argmax", "softmax"])
+@pytest.mark.parametrize("shape,axis", [([0, 300000], 1), ([0, 70001], 1), ([300000, 0], 0), ([0, 100, 5], 1), ([3, 40000, 0], 1)])
+def test_reductions_of_no_lines_compile(shape, axis, kind):
+    """An empty batch has no line to reduce, however long the axis: the layout rules divide by the
+    number of lines."""
+    g = Graph()
+    x = g.input(shape, DType.F32)
+    y = g.sum(x, axis) if kind == "sum" else g.argmax(x, axis) if kind == "argmax" else g.softmax(x, axis)
+    assert len(steps(g.codegen([y], compile=True))) == 1

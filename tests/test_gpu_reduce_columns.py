@@ -120,3 +120,12 @@ def test_column_softmax_and_rmsnorm_match_f64(hip):
     np.testing.assert_array_equal(ga.numpy(), gy.numpy().argmax(0))
     v64 = v.astype(np.float64)
     np.testing.assert_allclose(gr.numpy(), v64 / np.sqrt((v64 * v64).mean(0) + 1e-6), rtol=1e-5)
+
+
+@pytest.mark.parametrize("shape,axis", [((0, 300000), 1), ((300000, 0), 0), ((0, 100, 5), 1)])
+def test_reductions_of_no_lines_are_empty(hip, shape, axis):
+    """Long axes of an empty batch: no line, so no result."""
+    g = K.Graph()
+    x = g.input(shape, DType.F32)
+    y = g.softmax(x, axis)
+    check(hip, g, [g.sum(x, axis), g.argmax(x, axis), y], {x: Tensor(DType.F32, shape, b"")}, f"no lines {shape} axis {axis}")
