@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <stdexcept>
 
+#include "attention_row.h"
 #include "kernels.h"
 #include "numeric.h"
 
@@ -21,41 +22,11 @@ bool attention_f32_ok(const AttnArgs& a);
 
 namespace {
 
-// Sequences of a few positions and unaligned buffers: one thread per query row, online softmax in
-// registers. A serial chain over the keys, so its time grows with them.
+// Sequences of a few positions and unaligned buffers: one thread per query row.
 template <int D, int DT, class T>
 __global__ void __launch_bounds__(64) attn_rowwise_k(AttnArgs a) {
-  const int64_t head = blockIdx.y;
   const int64_t qi = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (qi >= a.s) return;
-  const T* Q = static_cast<const T*>(a.q) + head * a.s * D;
-  const T* K = static_cast<const T*>(a.k) + head * a.s * D;
-  const T* Vv = static_cast<const T*>(a.v) + head * a.s * D;
-  float q[D], acc[D];
-#pragma unroll
-  for (int t = 0; t < D; ++t) {
-    q[t] = load_elem<DT, T, float>(Q[qi * D + t]);
-    acc[t] = 0.f;
-  }
-  float m = -INFINITY, l = 0.f;
-  const int64_t kend = a.causal ? qi + 1 : a.s;
-  for (int64_t j = 0; j < kend; ++j) {
-    float sc = 0.f;
-#pragma unroll
-    for (int t = 0; t < D; ++t) sc = fmaf(q[t], load_elem<DT, T, float>(K[j * D + t]), sc);
-    sc *= a.scale;
-    float mn = fmaxf(m, sc);
-    float corr = expf(m - mn);
-    float p = expf(sc - mn);
-    l = l * corr + p;
-#pragma unroll
-    for (int t = 0; t < D; ++t) acc[t] = acc[t] * corr + p * load_elem<DT, T, float>(Vv[j * D + t]);
-    m = mn;
-  }
-  T* O = static_cast<T*>(a.o) + head * a.s * D;
-  const float inv = 1.f / l;
-#pragma unroll
-  for (int t = 0; t < D; ++t) O[qi * D + t] = store_elem<DT, T, float>(acc[t] * inv);
+  if (qi < a.s) attn_row<D, DT, T>(a, blockIdx.y, qi);
 }
 
 template <int D>

@@ -110,3 +110,43 @@ def test_f32_attention_with_minus_infinity_scores(hip, causal):
     with np.errstate(invalid="ignore"):  # the all -inf rows
         want = f64_attention(*(x.astype(np.float64) for x in (q, k, v)), causal)[0, 0]
     assert np.abs(got[lo:] - want[lo:]).max() <= 1e-5 * np.abs(want[lo:]).max()
+
+
+# (heads, positions): one tile a work-group; several, whose pipeline runs on into the next tile
+@pytest.mark.parametrize("h,s,grid", [(2, 150, None), (3, 300, "8")])
+@pytest.mark.parametrize("dt", [DType.BF16, DType.F16])
+@pytest.mark.parametrize("causal", [False, True])
+def test_16_bit_heads_of_32_with_infinities_and_nan_in_v(hip, monkeypatch, h, s, grid, dt, causal):
+    """Queries that see an infinity or NaN get it in its column, and f64's values in the others; other
+    heads keep their bits, and queries before it (causal) stay finite: they are within one rounding of
+    a run without it. The queries that met it are done again one to a thread: the bits of the kernel
+    for a few positions, which NO_MFMA selects."""
+    if grid:
+        monkeypatch.setenv("KURUMI_HIP_ATTN_GRID", grid)
+    p = s // 3
+    rng = np.random.default_rng(s)
+    arrays = [rng.standard_normal((3, h, s, 32)).astype(np.float32) for _ in range(3)]
+    arrays = [bf16_bits_to_f32(f32_to_bf16_bits(x)) if dt == DType.BF16 else x.astype(np.float16).astype(np.float32) for x in arrays]
+    q, k, v = arrays
+    clean = run(hip, dt, arrays, causal, "attn_mfma ")
+    v = v.copy()
+    v[1, 1, p + 1, 3], v[1, 1, p + 2, 4], v[1, 1, p + 20, 5] = np.inf, -np.inf, np.nan
+    got = run(hip, dt, [q, k, v], causal, "attn_mfma ")
+    monkeypatch.setenv("KURUMI_HIP_NO_MFMA", "1")
+    rows = run(hip, dt, [q, k, v], causal, "attn_rowwise")[1, 1]
+    other = np.ones((3, h), bool)
+    other[1, 1] = False
+    np.testing.assert_array_equal(got[other], clean[other])
+    got, clean = got[1, 1], clean[1, 1]
+    first = p + 20 if causal else 0  # the first query that sees all three
+    assert (got[first:, 3] == np.inf).all() and (got[first:, 4] == -np.inf).all() and np.isnan(got[first:, 5]).all()
+    np.testing.assert_array_equal(got[first:], rows[first:])
+    half_unit = 2.0 ** (-8 if dt == DType.BF16 else -11)
+    rest = [i for i in range(32) if i not in (3, 4, 5)]
+    scale = np.float32(32 ** -0.5)
+    scale = bf16_bits_to_f32(f32_to_bf16_bits(scale)) if dt == DType.BF16 else np.float16(scale)
+    want = f64_attention(*(x[1, 1].astype(np.float64) for x in arrays), causal, float(np.asarray(scale).item()))
+    assert np.abs(got[:, rest] - want[:, rest]).max() <= (half_unit + 2e-5) * np.abs(want).max()
+    if causal:
+        # both within half a unit in the last place of the largest (the other bar's bound) of f64
+        assert np.abs(got[:p + 1] - clean[:p + 1]).max() <= 2 * (half_unit + 2e-5) * np.abs(want).max()
