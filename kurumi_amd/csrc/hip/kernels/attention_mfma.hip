@@ -529,6 +529,8 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 bool attention_mfma_ok(const AttnArgs& a) {
   if (const char* e = std::getenv("KURUMI_HIP_NO_MFMA"); e && *e && *e != '0') return false;
   if (!(a.dtype == GT_BF16 || a.dtype == GT_F16)) return false;
+  // the maximum is taken over raw scores and masked ones are -inf before the scale: it must be positive
+  if (!(a.scale > 0.f && a.scale < 1e30f)) return false;
   if (!(a.d == 32 || a.d == 64 || a.d == 128)) return false;
   if (a.s <= 0 || a.bh <= 0 || a.bh * ((a.s + 127) / 128) > 0x7fffffff) return false;
   if (a.s * a.d * 2 >= (int64_t(1) << 31)) return false;  // per-head buffer offsets are 32-bit

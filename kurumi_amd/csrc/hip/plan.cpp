@@ -1843,7 +1843,7 @@ void Plan::compile() {
     } else {
       const AttnStep& A = attns_[s.index];
       AttnArgs a;
-      a.bh = (int64_t)A.bh; a.s = (int64_t)A.s; a.d = (int64_t)A.d; a.causal = A.causal; a.dtype = (int)A.dtype;
+      a.bh = (int64_t)A.bh; a.s = (int64_t)A.s; a.d = (int64_t)A.d; a.scale = A.scale; a.causal = A.causal; a.dtype = (int)A.dtype;
       std::ostringstream o;
       o << attn_variant(a) << " bh" << A.bh << " s" << A.s << " d" << A.d << (A.causal ? " causal" : "");
       s.label = o.str();

@@ -150,3 +150,36 @@ def test_16_bit_heads_of_32_with_infinities_and_nan_in_v(hip, monkeypatch, h, s,
     if causal:
         # both within half a unit in the last place of the largest (the other bar's bound) of f64
         assert np.abs(got[:p + 1] - clean[:p + 1]).max() <= 2 * (half_unit + 2e-5) * np.abs(want).max()
+
+
+@pytest.mark.parametrize("scale", [-0.375, 0.0])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dt,d,s", [(DType.BF16, 32, 100), (DType.F16, 32, 70), (DType.BF16, 64, 100), (DType.F16, 128, 70), (DType.F32, 32, 100)])
+def test_decomposed_attention_with_a_scale_that_is_not_positive(hip, dt, d, s, causal, scale):
+    """The chain softmax(q k^T * c) v takes any constant c. Bars as above, whatever the head size: in 16
+    bits such a scale takes the one-query-per-thread kernel, whose scores and probabilities are f32."""
+    rng = np.random.default_rng(s)
+    arrays = [rng.standard_normal((1, 2, s, d)).astype(np.float32) for _ in range(3)]
+    if dt == DType.BF16:
+        arrays = [bf16_bits_to_f32(f32_to_bf16_bits(x)) for x in arrays]
+        mk = lambda x: Tensor(dt, x.shape, f32_to_bf16_bits(x).tobytes())
+    elif dt == DType.F16:
+        arrays = [x.astype(np.float16).astype(np.float32) for x in arrays]
+        mk = lambda x: Tensor(dt, x.shape, x.astype(np.float16).tobytes())
+    else:
+        mk = Tensor.from_numpy
+    g = K.Graph()
+    ids = [g.input(x.shape, dt) for x in arrays]
+    raw = g.dot_general(ids[0], ids[1], [3], [3], [0, 1], [0, 1])
+    sc = g.mul(raw, g.scalar(raw, scale))
+    if causal:
+        mask = g.expand(g.reshape(g.constant(np.triu(np.full((s, s), -np.inf, np.float32), 1)), [1, 1, s, s]), [1, 2, s, s])
+        sc = g.add(sc, mask if dt == DType.F32 else g.cast(mask, dt))
+    o = g.dot_general(g.softmax(sc, 3), ids[2], [3], [2], [0, 1], [0, 1])
+    plan = hip.plan(g, [o], {i: mk(x) for i, x in zip(ids, arrays)})
+    assert len(plan.steps()) == 1 and plan.steps()[0].startswith("attn"), plan.steps()
+    plan.launch()
+    got = to_f32(plan.output(0))
+    want = f64_attention(*(x.astype(np.float64) for x in arrays), causal, scale)
+    half_unit = {DType.BF16: 2.0 ** -8, DType.F16: 2.0 ** -11, DType.F32: 0.0}[dt]
+    assert np.abs(got - want).max() <= (half_unit + 2e-5) * np.abs(want).max()
