@@ -1126,8 +1126,7 @@ void Planner::visit_quant(NodeId id) {
            : quant_mm_ok(qa)        ? QuantStep::MFMA
            : quant_flex_better(qa) ? QuantStep::FUSED_GEMM
                                     : QuantStep::DEQUANT_GEMM;
-  if (Q.path == QuantStep::FUSED_GEMM && quant_flex_scratch_bytes(qa))
-    Q.mm_slot = new_slot(SlotKind::Temp, DType::U8, quant_flex_scratch_bytes(qa), id);
+  Q.flex_scratch = Q.path == QuantStep::FUSED_GEMM ? quant_flex_scratch_bytes(qa) : 0;
   if (Q.path == QuantStep::DEQUANT_GEMM)
     Q.wdq_slot = new_slot(SlotKind::Temp, Q.wdq_dtype, Q.n * Q.k * dt_width(Q.wdq_dtype), id);
   if (Q.path == QuantStep::MFMA) {
@@ -1834,6 +1833,8 @@ void Plan::compile() {
         a.a = reinterpret_cast<const char*>(256) + Q.act_off * (int64_t)dt_width(Q.act_dtype);
         a.b = reinterpret_cast<const char*>(256);
         Q.ws_slot = scratch_slot(gemm_scratch_bytes(a));
+      } else if (Q.path == QuantStep::FUSED_GEMM) {
+        Q.ws_slot = scratch_slot(Q.flex_scratch);
       }
       std::ostringstream o;
       o << (Q.path == QuantStep::GEMV ? "quant_gemv" : Q.path == QuantStep::MFMA ? "quant_mfma" : Q.path == QuantStep::FUSED_GEMM ? "quant_dequant+gemm_fused" : "quant_dequant+gemm")
@@ -1851,14 +1852,17 @@ void Plan::compile() {
   }
 }
 
-// A scratch buffer of the plan for one of its steps; -1 where none is needed.
+// Scratch for one of the plan's steps (-1 where none is needed): one buffer of the largest size for
+// all of them, which run one after another on one stream.
 int Plan::scratch_slot(size_t bytes) {
   if (!bytes) return -1;
-  Slot s;
-  s.dtype = DType::U8;
-  s.bytes = bytes;
-  slots_.push_back(std::move(s));
-  return (int)slots_.size() - 1;
+  if (scratch_ < 0) {
+    scratch_ = (int)slots_.size();
+    slots_.emplace_back();
+    slots_.back().dtype = DType::U8;
+  }
+  slots_[scratch_].bytes = std::max(slots_[scratch_].bytes, bytes);
+  return scratch_;
 }
 
 // A step's GEMM without its addresses.
@@ -1990,7 +1994,7 @@ void Plan::launch_step(const Step& s) {
       }
       launch_quant_mm(a, st);
     } else if (Q.path == QuantStep::FUSED_GEMM) {
-      if (Q.mm_slot >= 0) a.mm_scratch = slot_ptr(slots_, Q.mm_slot);
+      if (Q.ws_slot >= 0) a.mm_scratch = slot_ptr(slots_, Q.ws_slot);
       launch_quant_flex(a, st);
     } else {
       a.wdq = slot_ptr(slots_, Q.wdq_slot);

@@ -134,7 +134,8 @@ struct QuantStep {
   DType act_dtype = DType::BF16, wdq_dtype = DType::BF16;
   bool tile_const = false;
   const void* qw_tiled = nullptr;
-  int ws_slot = -1;  // scratch of the GEMM after a dequantisation
+  int ws_slot = -1;         // scratch of a split K: of the GEMM after a dequantisation or the fused one
+  size_t flex_scratch = 0;  // what the latter needs
 };
 
 struct AttnStep {
@@ -239,6 +240,7 @@ class Plan {
   std::vector<ActqStep> actqs_;
   std::vector<Step> steps_;
   std::vector<int> order_;                 // execution order of steps
+  int scratch_ = -1;                       // slot of the steps' scratch
   std::map<NodeId, int> input_slots_;
   std::vector<std::pair<int, View>> root_vals_;  // slot + view of each root
   std::vector<std::string> sources_;

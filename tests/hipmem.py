@@ -63,3 +63,9 @@ class DevBuf:
 
 def synchronize() -> None:
     check(hip().hipDeviceSynchronize(), "hipDeviceSynchronize")
+
+
+def device_memory_free() -> int:
+    free, total = C.c_size_t(), C.c_size_t()
+    check(hip().hipMemGetInfo(C.byref(free), C.byref(total)), "hipMemGetInfo")
+    return free.value

@@ -6,6 +6,7 @@ import pytest
 
 import kurumi_amd as K
 from kurumi_amd import DType, Tensor
+from hipmem import device_memory_free
 from kutest import f32_to_bf16_bits, interpret, to_f32
 
 pytestmark = pytest.mark.gpu
@@ -103,3 +104,38 @@ def test_e4m3_products_of_few_tiles_match_oracle(hip, m, n, k):
     assert plan.steps()[-1].startswith("gemm_mfma_e4m3"), plan.steps()
     plan.launch()
     np.testing.assert_array_equal(plan.output(0).numpy(), interpret(g, [y], feeds)[0].numpy())
+
+
+def test_steps_of_a_plan_share_their_scratch():
+    """Split products, dequantising products and split reductions leave partial sums in one buffer of
+    the largest size, not in one each: the device memory that a plan of 33 such steps takes, and its results."""
+    count, m, n, k = 16, 32, 4096, 8192
+    rng = np.random.default_rng(11)
+    a = (rng.integers(-4, 5, (count * m, k)) / 8).astype(np.float32)
+    b = (rng.integers(-4, 5, (k, n)) / 8).astype(np.float32)
+    q = rng.integers(0, 256, (n, k // 2)).astype(np.uint8)
+    scale = np.full((n, k // 64), 0.25, np.float16)
+    hip = K.HipBackend()
+    g = K.Graph()
+    x, w = g.input(a.shape, DType.F32), g.input(b.shape, DType.F32)
+    qw = g.constant_bytes(DType.U8, q.tobytes(), list(q.shape))
+    sc = g.constant_bytes(DType.F16, scale.tobytes(), list(scale.shape))
+    parts = [g.slice(x, [(m * i, m * i + m), (0, k)]) for i in range(count)]
+    roots = [g.matmul(p, w) for p in parts] + [g.quant_matmul(p, qw, sc, None, 4, 64) for p in parts] + [g.sum(x, 0)]
+    feeds = {x: Tensor.from_numpy(a), w: Tensor.from_numpy(b)}
+    free = device_memory_free()
+    plan = hip.plan(g, roots, feeds)
+    taken = free - device_memory_free()
+    labels = plan.steps()
+    assert sum("_split" in s for s in labels) == count, labels
+    plan.launch()
+    got = [plan.output(i).numpy() for i in range(2 * count + 1)]
+    np.testing.assert_array_equal(np.concatenate(got[:count]), a @ b)  # sums of few 64ths: exact in any order
+    wq = np.stack([(q & 15).astype(np.int8), (q >> 4).astype(np.int8)], -1).reshape(n, k)
+    wq = np.where(wq > 7, wq - 16, wq).astype(np.float32) * 0.25
+    np.testing.assert_array_equal(np.concatenate(got[count:-1]), a @ wq.T)
+    np.testing.assert_array_equal(got[-1], a.sum(0))
+    partial = m * n * 4 * int(labels[0].split("_split")[1].split()[0])  # of one product
+    outs, ins = (2 * count * m * n + k) * 4, a.nbytes + b.nbytes + q.nbytes + scale.nbytes
+    print(f"taken {taken} inputs {ins} outputs {outs} partial sums {partial}", flush=True)
+    assert taken <= ins + outs + 8 * partial
