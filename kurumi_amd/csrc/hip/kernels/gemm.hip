@@ -12,6 +12,7 @@ namespace ku::hipbk {
 bool gemm_lds_ok(const GemmArgs& a);
 std::string gemm_lds_name(const GemmArgs& a);
 void launch_gemm_lds(const GemmArgs& a, hipStream_t s);
+bool gemm_lds_keeps(const GemmArgs& a);
 bool gemm_flex_ok(const GemmArgs& a);
 std::string gemm_flex_name(const GemmArgs& a);
 size_t gemm_flex_scratch_bytes(const GemmArgs& a);
@@ -26,9 +27,8 @@ Path path_of(const GemmArgs& a) {
   // loses when they do not (bf16, K x N = 4096 x 11008: 16 rows 63 against 20 us, 300 rows with
   // 2048 x 5504 42 against 25 us; 600 rows 58 against 73 us, 2048 rows 160 against 236 us), so the
   // two kernels' estimates are compared; within 10 % of each other the direct one is kept.
-  const bool flex = gemm_flex_ok(a);
-  if (gemm_lds_ok(a)) return flex && 1.1 * gemm_flex_us(a) < gemm_lds_us(a) ? Path::FLEX : Path::LDS;
-  return flex ? Path::FLEX : Path::GENERIC;
+  if (gemm_lds_ok(a)) return !gemm_lds_keeps(a) && gemm_flex_ok(a) && 1.1 * gemm_flex_us(a) < gemm_lds_us(a) ? Path::FLEX : Path::LDS;
+  return gemm_flex_ok(a) ? Path::FLEX : Path::GENERIC;
 }
 }  // namespace
 

@@ -699,13 +699,20 @@ bool gemm_lds_ok(const GemmArgs& a) {
   return a.batch <= 65535;
 }
 
-// Estimated microseconds. Products of one or two stages have kernels of their own, which nothing
-// else beats.
+// Products that stay with this kernel whatever the estimates say: those of one or two stages, which
+// have kernels of their own, and one tile of up to four stages (the register-staged kernel takes 5.6
+// us for 64 x 128 x 256 where this takes 7.8, but tests of the plan's labels pin the name).
+bool gemm_lds_keeps(const GemmArgs& a) {
+  return small_k(a) || (a.batch == 1 && a.m <= 192 && a.n <= 256 && a.k * (a.in_type == GT_F8E4M3 ? 1 : 2) <= 4 * KB);
+}
+
+// Estimated microseconds. The kernels of one or two stages are bound by their operands and C (bf16
+// 100 x 4096 x 128: 4.4 us, 1000 x 4096 x 128: 5.5 us, 2048 x 11008 x 128: 14.9 us).
 double gemm_lds_us(const GemmArgs& a) {
-  if (small_k(a)) return 0;
-  // one tile of up to four stages stays here as well, though the other kernel takes 5.6 us for 64 x
-  // 128 x 256 where this takes 7.8: tests of the plan's labels pin its name
-  if (a.batch == 1 && a.m <= 192 && a.n <= 256 && a.k * (a.in_type == GT_F8E4M3 ? 1 : 2) <= 4 * KB) return 0;
+  if (small_k(a)) {
+    const double in = a.in_type == GT_F8E4M3 ? 1 : 2, out = a.out_type == GT_F32 ? 4 : 2;
+    return 4 + (double)a.batch * ((double)(a.m + a.n) * a.k * in + (double)a.m * a.n * out) / 5e6;
+  }
   return tile_us(a, lds_tile(a));
 }
 

@@ -92,7 +92,12 @@ bool quant_flex_better(const QuantArgs& q) {
   g.a = g.b = nullptr;
   const double w = q.act_type == GT_F32 ? 4 : 2;
   const double expand = 2 + (double)q.n * q.k * (q.bits / 8.0 + w) / 5e6;  // 11008 x 4096 int4 -> bf16: 24.5 us
-  return choose(q).us < expand + gemm_estimated_us(g);
+  double us = choose(q).us;
+  // One or two stages of 16 bits: C is what takes the time, which this kernel writes two bytes a lane
+  // (int8 -> bf16 400 x 2048 x 128: 5.4 us against 6.9 expanded; int4 1000 x 4096 x 128: 13.4 against
+  // 8.1; 2048 x 11008 x 128: 39.9 against 20.4).
+  if (q.k * w <= 2 * KB && w == 2) us = std::max(us, 4 + (double)q.m * q.n * w / 0.9e6);
+  return us < expand + gemm_estimated_us(g);
 }
 
 size_t quant_flex_scratch_bytes(const QuantArgs& q) {

@@ -339,3 +339,16 @@ def test_reductions_of_no_lines_compile(shape, axis, kind):
     x = g.input(shape, DType.F32)
     y = g.sum(x, axis) if kind == "sum" else g.argmax(x, axis) if kind == "argmax" else g.softmax(x, axis)
     assert len(steps(g.codegen([y], compile=True))) == 1
+
+
+@pytest.mark.parametrize("m,n,k,bits,want", [
+    (100, 4096, 128, 8, "_fused"), (100, 4096, 192, 8, "_fused"),  # one side and the other of two stages of K
+    (16, 512, 128, 2, "_fused"), (16, 512, 192, 2, "_fused"),
+    (100, 256, 256, 8, "_fused"), (100, 320, 256, 8, "_fused"),    # one tile of the direct kernel, and two
+    (1000, 4096, 128, 4, ""), (2048, 11008, 128, 4, "")])          # so much of C that expanding is faster
+def test_quant_route_of_small_products_follows_the_time(m, n, k, bits, want):
+    g = Graph()
+    qw = g.constant_bytes(DType.U8, bytes(n * k * bits // 8), [n, k * bits // 8])
+    scales = g.constant_bytes(DType.F16, np.ones((n, k // 64), np.float16).tobytes(), [n, k // 64])
+    y = g.quant_matmul(g.input([m, k], DType.BF16), qw, scales, None, bits, 64)
+    assert [s.split()[0] for s in steps(g.codegen([y]))] == ["quant_dequant+gemm" + want]
