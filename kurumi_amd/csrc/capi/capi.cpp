@@ -682,10 +682,11 @@ int32_t ku_hip_linear_e4m3(const KuBackend* b, const void* x, uint32_t x_dtype, 
     a.k = (int64_t)k;
     auto& ctx = b->b->ctx();
     ctx.make_current();
-    const size_t need = ku::hipbk::linear_e4m3_scratch_bytes(a.m, a.n, a.k);
+    const ku::hipbk::GemmRoute route = ku::hipbk::linear_e4m3_route(a.m, a.n, a.k);
+    const size_t need = ku::hipbk::linear_e4m3_scratch_bytes(a.m, a.n, a.k, route);
     void* ws = b->b->workspace(need);
     try {
-      ku::hipbk::linear_e4m3(a, ws, need, stream ? static_cast<hipStream_t>(stream) : ctx.stream());
+      ku::hipbk::linear_e4m3(a, route, ws, need, stream ? static_cast<hipStream_t>(stream) : ctx.stream());
     } catch (const std::runtime_error& e) {
       throw ku::Error(std::string("ku_hip_linear_e4m3: ") + e.what());
     }

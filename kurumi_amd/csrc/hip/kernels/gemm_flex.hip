@@ -93,12 +93,8 @@ double gemm_flex_cost(const GemmArgs& a, int tile, int64_t splits, double extra,
   return us;
 }
 
-namespace {
-
-struct FlexPlan { int tile; int64_t splits; double us; };
-
-FlexPlan flex_plan(const GemmArgs& a) {
-  FlexPlan best{2, 1, 1e30};
+GemmRoute gemm_flex_route(const GemmArgs& a) {
+  GemmRoute best{GemmPath::FLEX, 2, 1, 1e30};
   const int64_t kt = stages(a);
   for (int i = 0; i < 3; ++i) {
     if (i < 2 && kTiles[i].bm >= 2 * a.m) continue;  // more than half of the tile's rows past M
@@ -109,13 +105,11 @@ FlexPlan flex_plan(const GemmArgs& a) {
           (uint64_t)(a.batch * (s * a.m * a.n * 4 + a.m * a.k)) > kLinearE4m3ScratchBytes - 8192)
         break;
       const double us = gemm_flex_cost(a, i, s, 0, (double)(a.k * a.n) * a.batch * width(a));
-      if (us < best.us) best = {i, s, us};
+      if (us < best.us) best = {GemmPath::FLEX, i, s, us};
     }
   }
   return best;
 }
-
-}  // namespace
 
 bool gemm_flex_ok(const GemmArgs& a) {
   if (const char* e = std::getenv("KURUMI_HIP_NO_MFMA"); e && *e && *e != '0') return false;
@@ -131,16 +125,7 @@ bool gemm_flex_ok(const GemmArgs& a) {
   return a.batch <= 65535 && (a.m + 31) / 32 * ((a.n + 63) / 64) < ((int64_t)1 << 24);
 }
 
-// Estimated microseconds of the launch (gemm.hip compares it with the direct-to-LDS kernel's).
-double gemm_flex_us(const GemmArgs& a) { return flex_plan(a).us; }
-
-size_t gemm_flex_scratch_bytes(const GemmArgs& a) {
-  const FlexPlan p = flex_plan(a);
-  return p.splits > 1 ? (size_t)(p.splits * a.batch * a.m * a.n) * 4 : 0;
-}
-
-std::string gemm_flex_name(const GemmArgs& a) {
-  const FlexPlan p = flex_plan(a);
+std::string gemm_flex_name(const GemmArgs& a, const GemmRoute& p) {
   std::string n = a.in_type == GT_F8E4M3 ? "gemm_mfma_e4m3" : a.in_type == GT_F32 ? "gemm_mfma_f32" : a.in_type == GT_F16 ? "gemm_mfma_f16" : "gemm_mfma_bf16";
   n += a.sbk == 1 ? "_nt_" : "_nn_";
   n += std::to_string(kTiles[p.tile].bm) + "x" + std::to_string(kTiles[p.tile].bn) + "_flex";
@@ -148,8 +133,10 @@ std::string gemm_flex_name(const GemmArgs& a) {
   return n;
 }
 
-// one tile shape and split (launch_gemm_flex picks them)
-void launch_gemm_flex_as(const GemmArgs& a, int tile, int64_t splits, hipStream_t s) {
+void launch_gemm_flex(const GemmArgs& a, const GemmRoute& r, hipStream_t s) {
+  const bool room = a.ws && a.ws_bytes >= gemm_scratch_bytes(a, r);
+  const int tile = r.tile;
+  const int64_t splits = room ? r.splits : 1;
   FlexArgs f{};
   f.g = a;
   f.part = static_cast<float*>(a.ws);
@@ -169,12 +156,6 @@ void launch_gemm_fold(const void* flex_args, hipStream_t s) {
   const int64_t total = f.g.batch * f.g.m * f.g.n;
   if (total % 4 == 0) hipLaunchKernelGGL((gemm_fold_k<4>), dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, s, f);
   else hipLaunchKernelGGL((gemm_fold_k<1>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, f);
-}
-
-void launch_gemm_flex(const GemmArgs& a, hipStream_t s) {
-  const FlexPlan p = flex_plan(a);
-  const bool room = a.ws && a.ws_bytes >= (size_t)(p.splits * a.batch * a.m * a.n) * 4;
-  launch_gemm_flex_as(a, p.tile, p.splits > 1 && room ? p.splits : 1, s);
 }
 
 }  // namespace ku::hipbk

@@ -50,14 +50,14 @@ void launch_bits(const FlexArgs& f, int bits, bool sym, int tile, hipStream_t s)
   }
 }
 
-struct Choice { int tile; int64_t splits; double us; };
+}  // namespace
 
-Choice choose(const QuantArgs& q) {
+GemmRoute quant_flex_route(const QuantArgs& q) {
   const GemmArgs a = as_gemm(q);
   const bool is32 = q.act_type == GT_F32;
   const int64_t kt = (q.k * (is32 ? 4 : 2) + KB - 1) / KB;
   const double b_bytes = (double)q.n * q.k * q.bits / 8;
-  Choice best{2, 1, 1e30};
+  GemmRoute best{GemmPath::FLEX, 2, 1, 1e30};
   for (int i = 0; i < 3; ++i) {
     if (i < 2 && kTiles[i].bm >= 2 * q.m) continue;
     // dequantising a stage of B: about 4.5 instructions a value on 64 lanes a clock, as much again
@@ -65,13 +65,11 @@ Choice choose(const QuantArgs& q) {
     const double extra = kTiles[i].bn * 64 * 4.5 / 64 / 2100;
     for (int64_t s = 1; s <= 64 && (s == 1 || kt / s >= 2); s *= 2) {
       const double us = gemm_flex_cost(a, i, s, extra, b_bytes);
-      if (us < best.us) best = {i, s, us};
+      if (us < best.us) best = {GemmPath::FLEX, i, s, us};
     }
   }
   return best;
 }
-
-}  // namespace
 
 bool quant_flex_ok(const QuantArgs& a) {
   if (const char* e = std::getenv("KURUMI_HIP_NO_MFMA"); e && *e && *e != '0') return false;
@@ -86,27 +84,24 @@ bool quant_flex_ok(const QuantArgs& a) {
 // multiplying: dequantising once per tile of rows beats the expanded weight's round trip up to a few
 // hundred rows (int4 -> bf16 11008 x 4096: 16 rows 20 us against 49, 100 rows 35 against 60, 256
 // rows of int8 61 against 80; 1024 rows 151 against 127, 2048 rows 253 against 182).
-bool quant_flex_better(const QuantArgs& q) {
+bool quant_flex_better(const QuantArgs& q, const GemmRoute& r) {
   if (!quant_flex_ok(q)) return false;
   GemmArgs g = as_gemm(q);
   g.a = g.b = nullptr;
   const double w = q.act_type == GT_F32 ? 4 : 2;
   const double expand = 2 + (double)q.n * q.k * (q.bits / 8.0 + w) / 5e6;  // 11008 x 4096 int4 -> bf16: 24.5 us
-  double us = choose(q).us;
+  double us = r.us;
   // One or two stages of 16 bits: C is what takes the time, which this kernel writes two bytes a lane
   // (int8 -> bf16 400 x 2048 x 128: 5.4 us against 6.9 expanded; int4 1000 x 4096 x 128: 13.4 against
   // 8.1; 2048 x 11008 x 128: 39.9 against 20.4).
   if (q.k * w <= 2 * KB && w == 2) us = std::max(us, 4 + (double)q.m * q.n * w / 0.9e6);
-  return us < expand + gemm_estimated_us(g);
+  return us < expand + gemm_route(g).us;
 }
 
-size_t quant_flex_scratch_bytes(const QuantArgs& q) {
-  const Choice c = choose(q);
-  return c.splits > 1 ? (size_t)(c.splits * q.m * q.n) * 4 : 0;
-}
+size_t quant_flex_scratch_bytes(const QuantArgs& q, const GemmRoute& r) { return gemm_scratch_bytes(as_gemm(q), r); }
 
-void launch_quant_flex(const QuantArgs& q, hipStream_t s) {
-  Choice c = choose(q);
+void launch_quant_flex(const QuantArgs& q, const GemmRoute& r, hipStream_t s) {
+  GemmRoute c = r;
   if (c.splits > 1 && !q.mm_scratch) c.splits = 1;
   FlexArgs f{};
   f.g = as_gemm(q);

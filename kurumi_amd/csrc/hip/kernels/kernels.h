@@ -35,16 +35,25 @@ struct GemmArgs {
 // Compute units of the current device (cached on first use): sizes persistent grids and tile rounds.
 int cu_count();
 
-// Short name of the kernel variant that will run (for plan labels): the MFMA kernel's element
+// How a product runs, from its sizes, types, strides and the alignment of a.a / a.b (null: aligned).
+// A plan decides it once, a direct call at its head: weighing the tiles and splits takes up to half a
+// microsecond.
+enum class GemmPath { LDS, FLEX, GENERIC };
+struct GemmRoute {
+  GemmPath path = GemmPath::GENERIC;
+  int tile = 0;        // FLEX: tile shape
+  int64_t splits = 1;  // FLEX: slices of K
+  double us = 1e9;     // estimated time
+};
+GemmRoute gemm_route(const GemmArgs& a);
+// Short name of the route's kernel (for plan labels): the MFMA kernel's element
 // type, layout and tile ("gemm_mfma_bf16_nn_256x256"; "_a64" when an operand spans 2^31 bytes or
 // more and the 64-bit-address DMA form runs), the
 // register-staged kernel's "gemm_mfma_<type>_<layout>_<tile>_flex[_split<n>]", or "gemm_generic".
-std::string gemm_variant(const GemmArgs& a);
-// scratch that the variant uses (0 for most); `a.a` / `a.b` need the alignment of the operands only
-size_t gemm_scratch_bytes(const GemmArgs& a);
-// estimated microseconds of the variant that will run
-double gemm_estimated_us(const GemmArgs& a);
-void launch_gemm(const GemmArgs& a, hipStream_t s);
+std::string gemm_variant(const GemmArgs& a, const GemmRoute& r);
+// scratch that the route uses (0 for most)
+size_t gemm_scratch_bytes(const GemmArgs& a, const GemmRoute& r);
+void launch_gemm(const GemmArgs& a, const GemmRoute& r, hipStream_t s);
 
 struct AttnArgs {
   const void* q = nullptr;
@@ -95,9 +104,11 @@ void launch_quant_mm(const QuantArgs& a, hipStream_t s);
 // dequantisation inside the GEMM (gemm_quant.hip): groups of a multiple of 16, any M and act type;
 // mm_scratch: quant_flex_scratch_bytes() for a split K, unsplit without it
 bool quant_flex_ok(const QuantArgs& a);
-bool quant_flex_better(const QuantArgs& a);
-size_t quant_flex_scratch_bytes(const QuantArgs& a);
-void launch_quant_flex(const QuantArgs& a, hipStream_t s);
+GemmRoute quant_flex_route(const QuantArgs& a);
+// whether it is the faster way than expanding the weight and multiplying
+bool quant_flex_better(const QuantArgs& a, const GemmRoute& r);
+size_t quant_flex_scratch_bytes(const QuantArgs& a, const GemmRoute& r);
+void launch_quant_flex(const QuantArgs& a, const GemmRoute& r, hipStream_t s);
 
 // Per-tensor e4m3 activation quantisation (linear_e4m3.hip): sx = max|x| * (1/448) and
 // xq = e4m3(x * (1/sx)) over n contiguous elements, in two kernels (absmax partials, then fold
@@ -125,11 +136,13 @@ struct LinearE4m3Args {
   int y_type = GT_BF16;
   int64_t m = 0, n = 0, k = 0;
 };
-// bytes of scratch one call needs: absmax partials, sx and the quantised activation (M*K); with n,
-// the GEMM's own scratch too (without room for it K is not split)
+// the route of its product
+GemmRoute linear_e4m3_route(int64_t m, int64_t n, int64_t k);
+// bytes of scratch one call needs: absmax partials, sx and the quantised activation (M*K); with n and
+// the route, the product's own scratch too (without room for it K is not split)
 size_t linear_e4m3_scratch_bytes(int64_t m, int64_t k);
-size_t linear_e4m3_scratch_bytes(int64_t m, int64_t n, int64_t k);
-void linear_e4m3(const LinearE4m3Args& a, void* scratch, size_t scratch_bytes, hipStream_t s);
+size_t linear_e4m3_scratch_bytes(int64_t m, int64_t n, int64_t k, const GemmRoute& r);
+void linear_e4m3(const LinearE4m3Args& a, const GemmRoute& r, void* scratch, size_t scratch_bytes, hipStream_t s);
 // The same with scratch in a static device array of kLinearE4m3ScratchBytes per GPU (no
 // allocation): m * k <= kLinearE4m3ScratchBytes - 4352. init_ looks the array up on the current GPU.
 constexpr size_t kLinearE4m3ScratchBytes = (size_t(16) << 20) + 4352;

@@ -241,7 +241,7 @@ GemmArgs linear_gemm(int64_t m, int64_t n, int64_t k) {
 }
 
 // `ws`: what is left of the scratch, for a split K
-void run_linear(const LinearE4m3Args& a, uint8_t* xq, float* partials, float* sx, void* ws, size_t ws_bytes, hipStream_t s) {
+void run_linear(const LinearE4m3Args& a, const GemmRoute& r, uint8_t* xq, float* partials, float* sx, void* ws, size_t ws_bytes, hipStream_t s) {
   ActQArgs q;
   q.x = a.x;
   q.x_type = a.x_type;
@@ -260,7 +260,7 @@ void run_linear(const LinearE4m3Args& a, uint8_t* xq, float* partials, float* sx
   g.alpha = sx;
   g.col_scale = a.sw;
   g.col_scale_stride = 1;
-  launch_gemm(g, s);
+  launch_gemm(g, r, s);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw std::runtime_error(std::string("launch failed: ") + hipGetErrorString(e));
 }
@@ -302,17 +302,19 @@ size_t linear_e4m3_scratch_bytes(int64_t m, int64_t k) { return kXqOff + (size_t
 // a split K's partial sums follow xq, 256-byte aligned
 static size_t partial_sums_off(int64_t m, int64_t k) { return (linear_e4m3_scratch_bytes(m, k) + 255) / 256 * 256; }
 
-size_t linear_e4m3_scratch_bytes(int64_t m, int64_t n, int64_t k) {
-  return partial_sums_off(m, k) + gemm_scratch_bytes(linear_gemm(m, n, k));
+GemmRoute linear_e4m3_route(int64_t m, int64_t n, int64_t k) { return gemm_route(linear_gemm(m, n, k)); }
+
+size_t linear_e4m3_scratch_bytes(int64_t m, int64_t n, int64_t k, const GemmRoute& r) {
+  return partial_sums_off(m, k) + gemm_scratch_bytes(linear_gemm(m, n, k), r);
 }
 
-void linear_e4m3(const LinearE4m3Args& a, void* scratch_buf, size_t scratch_bytes, hipStream_t s) {
+void linear_e4m3(const LinearE4m3Args& a, const GemmRoute& r, void* scratch_buf, size_t scratch_bytes, hipStream_t s) {
   check_linear(a);
   if (!scratch_buf || scratch_bytes < linear_e4m3_scratch_bytes(a.m, a.k))
     throw std::runtime_error("scratch buffer too small");
   uint8_t* base = static_cast<uint8_t*>(scratch_buf);
   const size_t used = std::min(partial_sums_off(a.m, a.k), scratch_bytes);
-  run_linear(a, base + kXqOff, reinterpret_cast<float*>(base + kPartialsOff), reinterpret_cast<float*>(base + kSxOff),
+  run_linear(a, r, base + kXqOff, reinterpret_cast<float*>(base + kPartialsOff), reinterpret_cast<float*>(base + kSxOff),
              base + used, scratch_bytes - used, s);
 }
 
@@ -324,7 +326,7 @@ void linear_e4m3_noalloc(const LinearE4m3Args& a, hipStream_t s) {
                              " bytes the static scratch holds for the quantised activation");
   uint8_t* base = scratch_on_current_device();
   const size_t used = std::min(partial_sums_off(a.m, a.k), kLinearE4m3ScratchBytes);
-  run_linear(a, base + kXqOff, reinterpret_cast<float*>(base + kPartialsOff), reinterpret_cast<float*>(base + kSxOff),
+  run_linear(a, linear_e4m3_route(a.m, a.n, a.k), base + kXqOff, reinterpret_cast<float*>(base + kPartialsOff), reinterpret_cast<float*>(base + kSxOff),
              base + used, kLinearE4m3ScratchBytes - used, s);
 }
 

@@ -1122,11 +1122,15 @@ void Planner::visit_quant(NodeId id) {
   // what the launch will see of the operands' addresses: buffers are 256-byte aligned
   qa.act = reinterpret_cast<const char*>(256) + Q.act_off * (int64_t)dt_width(at);
   qa.qw = reinterpret_cast<const uint8_t*>(256) + Q.qw_off;
-  Q.path = quant_gemv_ok(qa)        ? QuantStep::GEMV
-           : quant_mm_ok(qa)        ? QuantStep::MFMA
-           : quant_flex_better(qa) ? QuantStep::FUSED_GEMM
-                                    : QuantStep::DEQUANT_GEMM;
-  Q.flex_scratch = Q.path == QuantStep::FUSED_GEMM ? quant_flex_scratch_bytes(qa) : 0;
+  if (quant_gemv_ok(qa)) {
+    Q.path = QuantStep::GEMV;
+  } else if (quant_mm_ok(qa)) {
+    Q.path = QuantStep::MFMA;
+  } else {
+    Q.route = quant_flex_route(qa);
+    Q.path = quant_flex_better(qa, Q.route) ? QuantStep::FUSED_GEMM : QuantStep::DEQUANT_GEMM;
+    if (Q.path == QuantStep::FUSED_GEMM) Q.flex_scratch = quant_flex_scratch_bytes(qa, Q.route);
+  }
   if (Q.path == QuantStep::DEQUANT_GEMM)
     Q.wdq_slot = new_slot(SlotKind::Temp, Q.wdq_dtype, Q.n * Q.k * dt_width(Q.wdq_dtype), id);
   if (Q.path == QuantStep::MFMA) {
@@ -1816,9 +1820,10 @@ void Plan::compile() {
       a.a = reinterpret_cast<const char*>(256) + G.a_off * (int64_t)dt_width(G.in_dtype);
       a.b = reinterpret_cast<const char*>(256) + G.b_off * (int64_t)dt_width(G.in_dtype);
       if (G.alpha_slot >= 0) a.alpha = reinterpret_cast<const float*>(16);
-      G.ws_slot = scratch_slot(gemm_scratch_bytes(a));
+      G.route = gemm_route(a);
+      G.ws_slot = scratch_slot(gemm_scratch_bytes(a, G.route));
       std::ostringstream o;
-      o << gemm_variant(a) << " b" << G.batch << " m" << G.m << " n" << G.n << " k" << G.k;
+      o << gemm_variant(a, G.route) << " b" << G.batch << " m" << G.m << " n" << G.n << " k" << G.k;
       if (G.out_dtype != G.in_dtype && G.alpha_slot < 0) o << " +cast " << dt_name(G.out_dtype);
       s.label = o.str();
     } else if (s.type == Step::ACTQ) {
@@ -1832,7 +1837,8 @@ void Plan::compile() {
         GemmArgs a = quant_gemm_args(Q);
         a.a = reinterpret_cast<const char*>(256) + Q.act_off * (int64_t)dt_width(Q.act_dtype);
         a.b = reinterpret_cast<const char*>(256);
-        Q.ws_slot = scratch_slot(gemm_scratch_bytes(a));
+        Q.route = gemm_route(a);
+        Q.ws_slot = scratch_slot(gemm_scratch_bytes(a, Q.route));
       } else if (Q.path == QuantStep::FUSED_GEMM) {
         Q.ws_slot = scratch_slot(Q.flex_scratch);
       }
@@ -1957,7 +1963,7 @@ void Plan::launch_step(const Step& s) {
                    a.a, a.b, a.c, (long long)a.sab, (long long)a.sam, (long long)a.sak, (long long)a.sbb,
                    (long long)a.sbk, (long long)a.sbn, (long long)a.batch, (long long)a.m, (long long)a.n,
                    (long long)a.k, a.in_type, a.out_type);
-    launch_gemm(a, st);
+    launch_gemm(a, G.route, st);
     KU_HIP(hipGetLastError());
     ctx_->profile().launches[(int)Kind::Gemm]++;
   } else if (s.type == Step::ACTQ) {
@@ -1995,7 +2001,7 @@ void Plan::launch_step(const Step& s) {
       launch_quant_mm(a, st);
     } else if (Q.path == QuantStep::FUSED_GEMM) {
       if (Q.ws_slot >= 0) a.mm_scratch = slot_ptr(slots_, Q.ws_slot);
-      launch_quant_flex(a, st);
+      launch_quant_flex(a, Q.route, st);
     } else {
       a.wdq = slot_ptr(slots_, Q.wdq_slot);
       launch_quant_dequant(a, st);
@@ -2006,7 +2012,7 @@ void Plan::launch_step(const Step& s) {
         g.ws = slot_ptr(slots_, Q.ws_slot);
         g.ws_bytes = slots_[Q.ws_slot].bytes;
       }
-      launch_gemm(g, st);
+      launch_gemm(g, Q.route, st);
     }
     KU_HIP(hipGetLastError());
     ctx_->profile().launches[(int)Kind::Gemm]++;

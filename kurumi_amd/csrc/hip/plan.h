@@ -115,6 +115,7 @@ struct GemmStep {
   // fused cast epilogue: round to round_dtype (the dot's bf16 / f16) before storing out_dtype;
   // F32 = no extra rounding
   DType round_dtype = DType::F32;
+  GemmRoute route;
   int ws_slot = -1;  // scratch of a split K
 };
 
@@ -136,6 +137,7 @@ struct QuantStep {
   const void* qw_tiled = nullptr;
   int ws_slot = -1;         // scratch of a split K: of the GEMM after a dequantisation or the fused one
   size_t flex_scratch = 0;  // what the latter needs
+  GemmRoute route;          // of either
 };
 
 struct AttnStep {
