@@ -548,6 +548,7 @@ void Gen::plan_layout() {
   // few lines: spread each over more threads (down to 2 chunks per thread) until the launch has
   // about 16 waves per CU to hide memory latency with
   while (t < 1024 && lines * t < ((uint64_t)1 << 18) && chunks >= 4 * t) t *= 2;
+  while (t < rem) t *= 2;  // the elements left over go one to a thread
   TPL = (int)t;
   NC = (int)((chunks + TPL - 1) / TPL);
   // lines of one wave or less share a 256-thread group; a line of several waves is its own group

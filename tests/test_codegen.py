@@ -1,5 +1,7 @@
 """Fusion planning and code generation on the CPU (no GPU): every hot-path graph lowers to the
 expected number of device steps and each generated kernel compiles for gfx950 with hipRTC."""
+import re
+
 import numpy as np
 import pytest
 
@@ -352,3 +354,14 @@ def test_quant_route_of_small_products_follows_the_time(m, n, k, bits, want):
     scales = g.constant_bytes(DType.F16, np.ones((n, k // 64), np.float16).tobytes(), [n, k // 64])
     y = g.quant_matmul(g.input([m, k], DType.BF16), qw, scales, None, bits, 64)
     assert [s.split()[0] for s in steps(g.codegen([y]))] == ["quant_dequant+gemm" + want]
+
+
+def test_elements_left_over_have_a_thread_each(monkeypatch):
+    """Rows of no whole vectors: the last elements go one to a thread, also where the tuning variable
+    asks for more chunks per thread than a row has."""
+    monkeypatch.setenv("KURUMI_HIP_LINE_CHUNKS", "100")
+    g = Graph()
+    src = g.codegen([g.sum(g.input([300000, 263], DType.BF16), 1)], compile=True)  # vectors of 8, 7 elements left over
+    threads = int(re.search(r"lane = threadIdx\.x % (\d+)u", src).group(1))
+    left = int(re.search(r"if \(lane < (\d+)u\)", src).group(1))
+    assert left == 7 and threads >= left
