@@ -10,7 +10,7 @@ import pytest
 
 import kurumi_amd as K
 from kurumi_amd import DType, Tensor
-from kutest import f32_to_bf16_bits, interpret
+from kutest import bf16_bits_to_f32, f32_to_bf16_bits, interpret, to_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -129,3 +129,36 @@ def test_reductions_of_no_lines_are_empty(hip, shape, axis):
     x = g.input(shape, DType.F32)
     y = g.softmax(x, axis)
     check(hip, g, [g.sum(x, axis), g.argmax(x, axis), y], {x: Tensor(DType.F32, shape, b"")}, f"no lines {shape} axis {axis}")
+
+
+# one to eight adjacent lines a thread, which take 16384 lines each: short columns with one thread a
+# line and their values in registers, long ones with up to 16 threads and 128 KB of LDS; a middle axis
+@pytest.mark.parametrize("shape,axis,dt", [((40, 32768), 0, DType.F32), ((12, 65536), 0, DType.F32), ((100, 65536), 0, DType.F32),
+                                           ((3, 30, 22000), 1, DType.F32), ((9, 131072), 0, DType.BF16), ((130, 131072), 0, DType.BF16),
+                                           ((130, 131080), 0, DType.BF16)])
+def test_column_softmax_rmsnorm_and_argmax_of_many_lines_match_f64(hip, shape, axis, dt):
+    """Several levels of reduction over several lines a thread. f32 at the bar of 1e-5; bf16 within one
+    rounding of the output (2^-8 of it, as its significands have 8 bits) and 1e-5."""
+    print(f"{dt.name} {shape} axis {axis}", flush=True)
+    rng = np.random.default_rng(sum(shape))
+    v = 2 * rng.standard_normal(shape, dtype=np.float32)
+    if dt == DType.BF16:
+        bits = f32_to_bf16_bits(v)
+        v, t = bf16_bits_to_f32(bits), Tensor(dt, shape, bits.tobytes())
+    else:
+        t = Tensor.from_numpy(v)
+    g = K.Graph()
+    x = g.input(shape, dt)
+    y = g.softmax(x, axis)
+    roots = [y, g.argmax(y, axis), g.rmsnorm(x, axis, 1e-6)]
+    plan = hip.plan(g, roots, {x: t})
+    plan.launch()
+    gy, ga, gr = (to_f32(plan.output(0)), plan.output(1).numpy(), to_f32(plan.output(2)))
+    v = v.astype(np.float64)
+    e = np.exp(v - v.max(axis, keepdims=True))
+    want = e / e.sum(axis, keepdims=True)
+    bar = 1e-5 + (2.0 ** -8 if dt == DType.BF16 else 0.0)
+    assert (np.abs(gy - want) <= bar * want).all()
+    np.testing.assert_array_equal(ga, gy.argmax(axis))
+    want = v / np.sqrt((v * v).mean(axis, keepdims=True) + 1e-6)
+    assert (np.abs(gr - want) <= bar * np.abs(want)).all()
