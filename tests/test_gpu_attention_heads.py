@@ -183,3 +183,23 @@ def test_decomposed_attention_with_a_scale_that_is_not_positive(hip, dt, d, s, c
     want = f64_attention(*(x.astype(np.float64) for x in arrays), causal, scale)
     half_unit = {DType.BF16: 2.0 ** -8, DType.F16: 2.0 ** -11, DType.F32: 0.0}[dt]
     assert np.abs(got - want).max() <= (half_unit + 2e-5) * np.abs(want).max()
+
+
+# several tiles a work-group: mirrored rounds and a partial last tile; the head-grouped order over two
+# rounds; the same over three; one head of many tiles
+@pytest.mark.parametrize("b,h,s,grid", [(2, 4, 300, "8"), (2, 8, 256, "16"), (1, 24, 200, "16"), (1, 3, 1500, "8")])
+@pytest.mark.parametrize("dt", [DType.BF16, DType.F16])
+@pytest.mark.parametrize("causal", [False, True])
+def test_16_bit_heads_of_32_over_several_tiles_match_f64(hip, monkeypatch, b, h, s, grid, dt, causal):
+    """Queries of standard deviation 6: scores of up to 30, so that the running maximum moves by more than
+    the lazy rescale's 2^8. An f32 score of 30 is off by 2^-19, which the exponential makes 2e-6 of a
+    probability; 1e-4 covers the sums, the remainders and the fused scale."""
+    monkeypatch.setenv("KURUMI_HIP_ATTN_GRID", grid)
+    rng = np.random.default_rng(s)
+    arrays = [rng.standard_normal((b, h, s, 32)).astype(np.float32) * np.float32(x) for x in (6.0, 1.0, 1.0)]
+    arrays = [bf16_bits_to_f32(f32_to_bf16_bits(x)) if dt == DType.BF16 else x.astype(np.float16).astype(np.float32) for x in arrays]
+    got = run(hip, dt, arrays, causal, "attn_mfma ")
+    scale = np.float32(32 ** -0.5)
+    scale = bf16_bits_to_f32(f32_to_bf16_bits(scale)) if dt == DType.BF16 else np.float16(scale)
+    want = f64_attention(*(x.astype(np.float64) for x in arrays), causal, float(np.asarray(scale).item()))
+    assert np.abs(got - want).max() <= (2.0 ** (-8 if dt == DType.BF16 else -11) + 1e-4) * np.abs(want).max()
