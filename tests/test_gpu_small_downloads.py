@@ -1,5 +1,6 @@
-"""Outputs on both sides of the size that goes through pinned memory, alone and from several threads
-with a backend each: whole bytes, so equality is exact."""
+"""Outputs on both sides of the size that goes through pinned memory: alone, from several threads with a
+backend each, and from several that share one backend and so its pinned buffer. Whole bytes, so
+equality is exact."""
 import threading
 
 import numpy as np
@@ -31,14 +32,20 @@ def test_output_bytes_arrive_whole(hip, n):
         check(plan, g, x, n, seed)
 
 
-def test_threads_each_get_their_own_bytes():
+@pytest.mark.parametrize("shared", [False, True])
+def test_threads_each_get_their_own_bytes(shared):
     sizes = (1000, 4096, 65536, 65537)
     wrong = []
+    plans = [None] * len(sizes)
+    if shared:  # planned and run once (which records each plan's graph) before the threads start
+        be = K.HipBackend()
+        for i, n in enumerate(sizes):
+            plans[i] = make(be, n)
+            check(plans[i][2], *plans[i][:2], n, i)
 
     def work(i):
         try:
-            be = K.HipBackend()
-            g, x, plan = make(be, sizes[i])
+            g, x, plan = plans[i] or make(K.HipBackend(), sizes[i])
             for seed in range(20):
                 check(plan, g, x, sizes[i], 100 * i + seed)
         except Exception as e:
