@@ -24,7 +24,7 @@ def sixteenths(rng, shape):
 
 
 # tiles cut by M, N and K, one element, one column, rows of odd length, whole tiles, long K on few
-# tiles (split), more rows than one tile of each height, aligned products of few tiles
+# tiles (split), many tiles, aligned products of few tiles
 SIZES = [(1, 1, 1), (2, 3, 5), (33, 1, 70), (1, 130, 129), (31, 65, 127), (64, 64, 64), (130, 129, 33), (7, 128, 2496),
          (257, 300, 95), (1030, 1400, 256), (5, 7, 9001), (200, 120, 1111), (16, 512, 1024), (300, 264, 2048)]
 
@@ -39,10 +39,27 @@ def test_products_of_any_size_match_oracle(hip, dt, nt, m, n, k):
     a, b = g.input([m, k], dt), g.input([n, k] if nt else [k, n], dt)
     y = g.dot_general(a, b, [1], [1 if nt else 0])
     feeds = {a: tensor(sixteenths(rng, (m, k)), dt), b: tensor(sixteenths(rng, (n, k) if nt else (k, n)), dt)}
-    assert "gemm_mfma" in hip.plan(g, [y], feeds).steps()[-1]
+    label = hip.plan(g, [y], feeds).steps()[-1].split()[0]
+    direct = dt != DType.F32 and (m, n, k) == (64, 64, 64)  # one stage of K: the direct-to-LDS kernel's
+    assert ("_flex" in label) != direct and ("_split" in label) == (k in (2496, 9001, 1111, 1024, 2048)), label
     roots = [y, g.cast(y, DType.F16 if dt != DType.F16 else DType.F32)]
     for r in roots:  # each alone: the cast rides in the product's epilogue
         np.testing.assert_array_equal(hip.eval_with(g, r, feeds).numpy(), interpret(g, [r], feeds)[0].numpy())
+
+
+@pytest.mark.parametrize("dt,m,n,k", [(DType.F32, 3041, 3719, 517), (DType.BF16, 907, 3331, 70), (DType.F16, 907, 3331, 70)])
+@pytest.mark.parametrize("nt", [False, True])
+def test_the_largest_tiles_match_numpy(hip, dt, m, n, k, nt):
+    """128 x 128 tiles, cut by M, N and K (the oracle would take a minute: numpy's f32 product, whose
+    sums are exact too)."""
+    rng = np.random.default_rng(m)
+    g = K.Graph()
+    a, b = g.input([m, k], dt), g.input([n, k] if nt else [k, n], dt)
+    x, w = sixteenths(rng, (m, k)), sixteenths(rng, (n, k) if nt else (k, n))
+    plan = hip.plan(g, [g.dot_general(a, b, [1], [1 if nt else 0])], {a: tensor(x, dt), b: tensor(w, dt)})
+    assert "_128x128_flex" in plan.steps()[0], plan.steps()
+    plan.launch()
+    np.testing.assert_array_equal(to_f32(plan.output(0)), to_f32(tensor(x @ (w.T if nt else w), dt)))
 
 
 @pytest.mark.parametrize("dt", [DType.F32, DType.BF16])
@@ -85,8 +102,9 @@ def test_f32_products_keep_infinities_nans_and_denormals(hip, m, n, k):
     np.testing.assert_array_equal(got, want)
 
 
-# few tiles, cut by M and N; one stage and many; split and unsplit; the last of the rows that take it
-@pytest.mark.parametrize("m,n,k", [(1, 64, 128), (33, 70, 256), (16, 512, 4096), (130, 100, 640), (300, 520, 384), (1024, 65, 128), (7, 3000, 2048)])
+# few tiles, cut by M and N, split and unsplit, the last of the rows that take it; one and two stages,
+# which the direct-to-LDS kernel keeps
+@pytest.mark.parametrize("m,n,k", [(1, 64, 128), (33, 70, 256), (16, 512, 4096), (130, 100, 640), (300, 520, 384), (1024, 65, 384), (1024, 65, 128), (7, 3000, 2048)])
 def test_e4m3_products_of_few_tiles_match_oracle(hip, m, n, k):
     """The e4m3 linear's product (operands multiples of 1/16, exact in e4m3, unit scales) in f32."""
     print(f"e4m3 {m}x{n}x{k}", flush=True)
@@ -101,7 +119,8 @@ def test_e4m3_products_of_few_tiles_match_oracle(hip, m, n, k):
     feeds = {a: Tensor(DType.F8E4M3, (m, k), rng.choice(codes, (m, k)).tobytes()), b: Tensor(DType.F8E4M3, (n, k), rng.choice(codes, (n, k)).tobytes()),
              sx: tensor([0.5], DType.F32), sw: tensor(2.0 ** rng.integers(-2, 3, n), DType.F32)}
     plan = hip.plan(g, [y], feeds)
-    assert plan.steps()[-1].startswith("gemm_mfma_e4m3"), plan.steps()
+    label = plan.steps()[-1].split()[0]
+    assert label.startswith("gemm_mfma_e4m3") and ("_flex" in label) == (k > 256) and ("_split" in label) == (k >= 2048), label
     plan.launch()
     np.testing.assert_array_equal(plan.output(0).numpy(), interpret(g, [y], feeds)[0].numpy())
 

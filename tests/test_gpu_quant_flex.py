@@ -37,7 +37,28 @@ def quant_case(rng, m, n, k, bits, group, sym, dt):
 def test_dequantising_gemm_matches_oracle(hip, m, n, k, group, bits, sym, dt):
     print(f"{dt.name} int{bits} sym={sym} {m}x{n}x{k} g{group}", flush=True)
     g, y, feeds = quant_case(np.random.default_rng(m + n + k), m, n, k, bits, group, sym, dt)
+    mfma = bits == 4 and 9 <= m <= 64 and group % 64 == 0 and dt != DType.F32  # the kernel for few rows of int4
+    assert hip.plan(g, [y], feeds).steps()[0].startswith("quant_mfma " if mfma else "quant_dequant+gemm_fused ")
     np.testing.assert_array_equal(hip.eval_with(g, y, feeds).numpy(), interpret(g, [y], feeds)[0].numpy())
+
+
+@pytest.mark.parametrize("m,n,k,bits,dt", [(163, 11065, 256, 4, DType.BF16), (163, 3001, 2048, 8, DType.F16), (66, 11065, 4096, 4, DType.F32)])
+def test_dequantising_gemm_of_the_largest_tiles_matches_numpy(hip, m, n, k, bits, dt):
+    """128 x 128 tiles cut by M and N, unsplit and split (the oracle would take minutes: numpy's f32
+    product, whose sums are exact too)."""
+    rng = np.random.default_rng(m)
+    g, y, feeds = quant_case(rng, m, n, k, bits, 64, True, dt)
+    plan = hip.plan(g, [y], feeds)
+    assert plan.steps()[0].startswith("quant_dequant+gemm_fused "), plan.steps()
+    plan.launch()
+    rng = np.random.default_rng(m)  # the same draws again
+    v = (rng.integers(-16, 17, (m, k)) / 16).astype(np.float32)
+    packed = rng.integers(0, 256, (n, k * bits // 8), dtype=np.uint8)
+    scales = (2.0 ** rng.integers(-6, -3, (n, k // 64))).astype(np.float32)
+    q = packed.astype(np.int8) if bits == 8 else np.stack([packed << 4, packed], -1).astype(np.int8).reshape(n, k) >> 4
+    want = v @ (q.astype(np.float32) * np.repeat(scales, 64, 1)).T
+    raw = f32_to_bf16_bits(want) if dt == DType.BF16 else want.astype(np.float16) if dt == DType.F16 else want
+    np.testing.assert_array_equal(plan.output(0).numpy(), Tensor(dt, (m, n), raw.tobytes()).numpy())
 
 
 @pytest.mark.parametrize("m,n,k,group,bits,dt,want", [
