@@ -489,8 +489,9 @@ void Gen::plan_layout() {
   // A line region's V and TPL fix the order its reductions add in, so they depend only on what
   // the reduced values are computed from (leaves, line length, the region's structure), never
   // on which values are stored: a node evaluated alone and within eval_many over several roots
-  // then gets the same bits (kurumi_core/tests/engine.rs:224-243). Flat regions (no reductions)
-  // size their vectors by their outputs too.
+  // then gets the same bits (kurumi_core/tests/engine.rs:224-243), unless another root adds nodes to
+  // its region (a sum, and x / sum beside it). Flat regions (no reductions) size their vectors by
+  // their outputs too.
   if (flat)
     for (auto& op : R.outputs) minw = std::min<int>(minw, (int)dt_width(node(op.first).dtype));
   V = std::min(8, 16 / std::max(minw, 1));
@@ -559,8 +560,9 @@ void Gen::plan_layout() {
 }
 
 // One level of reductions and nothing computed from them per element: the axis may be split over
-// work-groups. The rule looks at the region's structure only, not at what is stored, so a
-// reduction keeps its bits when it is evaluated with other outputs.
+// work-groups. The rule looks at the region's structure only, not at what is stored, so a reduction
+// keeps its bits whichever of the region's values are outputs. Beside a value computed from it per
+// element (x / sum(x)) it may add in another order than alone, as rows do (`full_out`).
 static bool splittable(const Region& R) {
   for (auto& n : R.nodes)
     if (n.level > 1 || (n.level == 1 && n.space == Space::Full)) return false;

@@ -145,11 +145,12 @@ attn_mfma_k(AttnArgs a) {
   constexpr int NBLK = TBYTES / 1024 / NW;  // 1 KB DMA blocks per wave per tile
   constexpr int DS = D / 16;             // k-steps of S^T
   constexpr int DTL = D / 32;            // 32-row tiles of O^T
-  // Heads of 32 keep the probabilities to 32-bit precision: a 16-bit value plus the 16-bit value of
-  // what its rounding left (2^-17 of a probability in bf16), a product each, and f32 row sums. The
-  // P.V product is a small part of a block there: bf16 [4, 4, 2986, 32]
-  // takes 51 us (45 without the remainders, at 1.35 times the error against f64), 2876 us on the
-  // one-query-per-thread kernel.
+  // Heads of 32 hold a probability as two 16-bit values, its rounding and the rounding of what that
+  // left, with a product each, and f32 row sums: to 2^-17 of itself in bf16 and 2^-22 in f16, where the
+  // one-query-per-thread kernel multiplies 24-bit ones. The output's own rounding (2^-9, 2^-12) covers
+  // the difference: the error against f64 is that kernel's within 0.01 % (5 to 4096 positions, queries of
+  // standard deviation 1 and 4). The P.V product is a small part of a block here: bf16 [4, 4, 2986, 32]
+  // takes 51 us (45 without the remainders, at 1.35 times the error), 2876 us on that kernel.
   constexpr bool SPLIT_P = D == 32;
   static_assert(W >= 1 && NBLK * NW * 1024 == TBYTES, "K / V staging");
   // every block a wave needs starts at or before the wave's first query, so a lane is never

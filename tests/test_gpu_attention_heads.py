@@ -4,7 +4,8 @@ softmax(q k^T / sqrt(d)) v in f64.
 Bars: f32 1e-5 of the largest output (the f32 bar used throughout; sums of up to 1000 terms of one
 sign and magnitude carry a few 2^-24); 16 bits one rounding of the output, half a unit in the last
 place of the largest output (at most 2^-8 of it in bf16, whose significands have 8 bits, 2^-11 in f16)
-and 2e-5 on top: the probabilities are kept to 32-bit precision."""
+and 2e-5 on top: the probabilities are two 16-bit values, within 2^-17 (f16: 2^-22) of themselves, and
+their sums f32."""
 import numpy as np
 import pytest
 
