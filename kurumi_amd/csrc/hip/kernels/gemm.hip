@@ -18,6 +18,7 @@ bool gemm_lds_keeps(const GemmArgs& a);
 bool gemm_flex_ok(const GemmArgs& a);
 GemmRoute gemm_flex_route(const GemmArgs& a);
 std::string gemm_flex_name(const GemmArgs& a, const GemmRoute& r);
+double gemm_flex_tiles_elements(const GemmArgs& a, const GemmRoute& r);
 double gemm_lds_us(const GemmArgs& a);
 void launch_gemm_flex(const GemmArgs& a, const GemmRoute& r, hipStream_t s);
 
@@ -34,6 +35,11 @@ GemmRoute gemm_route(const GemmArgs& a) {
   }
   if (!gemm_flex_ok(a)) return lds;
   const GemmRoute flex = gemm_flex_route(a);
+  // K within one 16-deep tile of the generic kernel, which a stage of the register-staged one, cut
+  // and loaded element by element, does not beat at any size (f32 500 x 500 x 16: 5.1 against 6.0 us,
+  // x 20: 6.9 against 6.0); up to twice that where writing C takes the time, which the generic kernel
+  // does faster (bf16 3000 x 4001 x 24: 21.7 against 25.4 us; 1000 x 2001 x 24: 8.4 against 7.5).
+  if (lds.path != GemmPath::LDS && (a.k <= 16 || (a.k < 32 && gemm_flex_tiles_elements(a, flex) >= 4e6))) return lds;
   return lds.path != GemmPath::LDS || 1.1 * flex.us < lds.us ? flex : lds;
 }
 

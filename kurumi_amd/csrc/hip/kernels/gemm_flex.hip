@@ -125,6 +125,12 @@ bool gemm_flex_ok(const GemmArgs& a) {
   return a.batch <= 65535 && (a.m + 31) / 32 * ((a.n + 63) / 64) < ((int64_t)1 << 24);
 }
 
+// elements of C that the route's tiles cover, those past M and N included
+double gemm_flex_tiles_elements(const GemmArgs& a, const GemmRoute& r) {
+  const Tile& t = kTiles[r.tile];
+  return (double)((a.m + t.bm - 1) / t.bm * t.bm) * (double)((a.n + t.bn - 1) / t.bn * t.bn) * (double)a.batch;
+}
+
 std::string gemm_flex_name(const GemmArgs& a, const GemmRoute& p) {
   std::string n = a.in_type == GT_F8E4M3 ? "gemm_mfma_e4m3" : a.in_type == GT_F32 ? "gemm_mfma_f32" : a.in_type == GT_F16 ? "gemm_mfma_f16" : "gemm_mfma_bf16";
   n += a.sbk == 1 ? "_nt_" : "_nn_";

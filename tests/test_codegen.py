@@ -365,3 +365,12 @@ def test_elements_left_over_have_a_thread_each(monkeypatch):
     threads = int(re.search(r"lane = threadIdx\.x % (\d+)u", src).group(1))
     left = int(re.search(r"if \(lane < (\d+)u\)", src).group(1))
     assert left == 7 and threads >= left
+
+
+@pytest.mark.parametrize("dt", [DType.F32, DType.BF16])
+@pytest.mark.parametrize("m,n,k,flex", [(1, 1, 1, False), (500, 500, 16, False), (500, 500, 17, True), (1000, 2001, 24, True),
+                                        (3000, 4001, 24, False), (3000, 4001, 40, True)])
+def test_products_of_a_short_k_take_the_generic_kernel(m, n, k, flex, dt):
+    g = Graph()
+    label = steps(g.codegen([g.matmul(g.input([m, k], dt), g.input([k, n], dt))]))[-1].split()[0]
+    assert ("_flex" in label) == flex and (label == "gemm_generic") != flex, label
