@@ -446,6 +446,16 @@ std::string Gen::op_expr(int ni, const std::string& j) const {
   }
 }
 
+// One level of reductions and nothing computed from them per element: the axis may be split over
+// work-groups. The rule looks at the region's structure only, not at what is stored, so a reduction
+// keeps its bits whichever of the region's values are outputs. Beside a value computed from it per
+// element (x / sum(x)) it may add in another order than alone, as rows do (`full_out`).
+static bool splittable(const Region& R) {
+  for (auto& n : R.nodes)
+    if (n.level > 1 || (n.level == 1 && n.space == Space::Full)) return false;
+  return true;
+}
+
 // Decide flat vs line layout, vector width, threads per line, chunks per thread.
 void Gen::plan_layout() {
   rank = (int)R.S.size();
@@ -495,11 +505,20 @@ void Gen::plan_layout() {
   if (flat)
     for (auto& op : R.outputs) minw = std::min<int>(minw, (int)dt_width(node(op.first).dtype));
   V = std::min(8, 16 / std::max(minw, 1));
-  // Long rows keep whole vectors at any length: the accesses need element alignment only, and the
-  // few elements left over take one more step (f32 [4, 50257] softmax + argmax, element by element
-  // from memory in every phase: 31.5 us; here 15.4 us, which is the arithmetic of one row on one CU).
-  // Short rows would gain nothing.
-  const bool any_length = !flat && !col && L >= 256;
+  // Rows of 256 elements and more whose length is no multiple of a vector: the widest vector that
+  // divides it (`even`), or whole vectors at element alignment and one more step for the few elements
+  // left over. Whole ones win where the narrow ones leave each thread of a full group more values than
+  // it keeps in registers, and where there are few rows, whose time is latency; with many shorter rows
+  // they lose. f32, narrow against whole: softmax + argmax [4, 50257] 31.5 / 15.4 us, [1000, 20001] 64 /
+  // 38, [300, 3001] 7.6 / 6.1, [3000, 7054] 31 / 48, [10000, 1033] 21 / 27; bf16: [300, 7054] 8.9 / 6.9,
+  // [3000, 5003] 24 / 18, [10000, 1498] 17 / 26, argmax of it 6.6 / 13.9. f32 sums, maxima and
+  // argmaxes with nothing computed from them per element take whole ones at any number of rows (argmax
+  // [1000, 1999] 5.0 / 3.4, sum [10000, 1033] 7.9 / 6.9).
+  uint64_t even = 1;
+  while (even < (uint64_t)V && L % (2 * even) == 0) even *= 2;
+  const bool whole = V == 8 ? L > 4 * 1024 * even || lines <= 1024
+                            : L > 12 * 1024 * even || lines <= 512 || (V == 4 && splittable(R));
+  const bool any_length = !flat && !col && L >= 256 && whole;
   while (V > 1 && !any_length && (R.S[vecaxis] % (uint64_t)V) != 0) V /= 2;
   if (any_length) rem = L % (uint64_t)V;
   mainV = V;
@@ -557,16 +576,6 @@ void Gen::plan_layout() {
   WG = TPL > 64 ? TPL : 256;
   GPW = WG / TPL;
   plan_split();
-}
-
-// One level of reductions and nothing computed from them per element: the axis may be split over
-// work-groups. The rule looks at the region's structure only, not at what is stored, so a reduction
-// keeps its bits whichever of the region's values are outputs. Beside a value computed from it per
-// element (x / sum(x)) it may add in another order than alone, as rows do (`full_out`).
-static bool splittable(const Region& R) {
-  for (auto& n : R.nodes)
-    if (n.level > 1 || (n.level == 1 && n.space == Space::Full)) return false;
-  return true;
 }
 
 // Threads of a column kernel. A wave reads CW * V consecutive elements of a row, so its loads

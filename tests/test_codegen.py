@@ -359,9 +359,9 @@ def test_quant_route_of_small_products_follows_the_time(m, n, k, bits, want):
 def test_elements_left_over_have_a_thread_each(monkeypatch):
     """Rows of no whole vectors: the last elements go one to a thread, also where the tuning variable
     asks for more chunks per thread than a row has."""
-    monkeypatch.setenv("KURUMI_HIP_LINE_CHUNKS", "100")
+    monkeypatch.setenv("KURUMI_HIP_LINE_CHUNKS", "1000")
     g = Graph()
-    src = g.codegen([g.sum(g.input([300000, 263], DType.BF16), 1)], compile=True)  # vectors of 8, 7 elements left over
+    src = g.codegen([g.sum(g.input([300000, 4103], DType.BF16), 1)], compile=True)  # vectors of 8, 7 elements left over
     threads = int(re.search(r"lane = threadIdx\.x % (\d+)u", src).group(1))
     left = int(re.search(r"if \(lane < (\d+)u\)", src).group(1))
     assert left == 7 and threads >= left
@@ -374,3 +374,15 @@ def test_products_of_a_short_k_take_the_generic_kernel(m, n, k, flex, dt):
     g = Graph()
     label = steps(g.codegen([g.matmul(g.input([m, k], dt), g.input([k, n], dt))]))[-1].split()[0]
     assert ("_flex" in label) == flex and (label == "gemm_generic") != flex, label
+
+
+@pytest.mark.parametrize("rows,cols,dt,vector", [
+    (10000, 1498, DType.BF16, 2), (3000, 7054, DType.F32, 2), (1025, 4095, DType.BF16, 1), (513, 12287, DType.F32, 1),  # what the length allows
+    (1024, 4095, DType.BF16, 8), (1025, 4097, DType.BF16, 8), (512, 12287, DType.F32, 4), (513, 12289, DType.F32, 4)])  # whole vectors and the rest
+def test_rows_of_odd_length_take_whole_vectors_where_few_or_long(rows, cols, dt, vector):
+    g = Graph()
+    x = g.input([rows, cols], dt)
+    y = g.softmax(x, 1)
+    kernel = g.codegen([y, g.argmax(y, 1)], compile=True).split("__global__")[1]
+    assert int(re.search(r"float f0\[(\d+)\]", kernel).group(1)) == vector
+    assert bool(re.search(r"if \(lane < \d+u\)", kernel)) == (vector == (4 if dt == DType.F32 else 8))  # the elements left over
