@@ -591,6 +591,18 @@ void Gen::plan_columns() {
   // groups (16 threads still read 64-byte segments of 4-byte elements)
   if (!split)
     while (V > 1 && lines / V < 64 * 256) V /= 2;
+  // Short columns have one thread or a few along the axis: where the lines alone do not fill the chip a
+  // vector of them only makes each thread's chain longer (bf16 softmax [16, 131072], eight lines a
+  // thread 8.1 us, one 3.4; f32 [16, 400000], four 8.8, one 10.4). So do the 8-byte indices of an
+  // argmax, whose stores scatter, and its folds through LDS (bf16 argmax [2, 3000000] 10.6 and 6.7 us,
+  // f32 [24, 8000] with two threads a line 4.2, one 3.2; not beside a sum, whose order would change).
+  bool arg = false, ordered = false;
+  for (auto& n : R.nodes) {
+    arg = arg || n.kind == (int)OpKind::ArgReduce;
+    ordered = ordered || n.kind == (int)OpKind::Sum || n.kind == (int)OpKind::Prod;
+  }
+  const bool few = lines / V < ((uint64_t)1 << 16);
+  if (L <= 16 ? few || (arg && (split || V == 8)) : L < 64 && split && arg && few) V = 1;
   const uint64_t nvl = (lines + V - 1) / V;
   CW = 64;
   while (CW > 1 && (uint64_t)CW / 2 >= nvl) CW /= 2;
@@ -599,8 +611,10 @@ void Gen::plan_columns() {
   const int most = split ? 256 : 1024;
   TPL = 1;
   // at least 8 rows per thread: short lines keep one thread each and their values in registers
-  while (CW * TPL < most && L > 16 && L / (2 * TPL) >= 8 && (CW * TPL < 64 || nvl * TPL < threads)) TPL *= 2;
-  WG = std::max(64, CW * TPL);
+  while (CW * TPL < most && L > (split && few && arg && !ordered ? 32 : 16) && L / (2 * TPL) >= 8 && (CW * TPL < 64 || nvl * TPL < threads)) TPL *= 2;
+  // one thread a line: larger groups where one-wave groups would come by the thousand (vectors of lines
+  // keep one-wave groups: f32 softmax [16, 400000] 8.7 us, 9.8 with 256 threads)
+  WG = TPL == 1 && V == 1 && nvl >= ((uint64_t)1 << 16) ? 256 : std::max(64, CW * TPL);
   CW = WG / TPL;
   GPW = CW;
   NC = (int)((L + TPL - 1) / TPL);
@@ -701,8 +715,9 @@ void Gen::schedule() {
     if (!std::getenv("KURUMI_HIP_LINE_WAVES")) min_waves = std::max(min_waves, std::min(8, 512 / (regs + 40)));
   }
   // loops along a column, and slices, hold nothing from one phase to the next
-  counted = !flat && cached.empty() && (col || Z > 1);
+  counted = !flat && cached.empty() && (col || Z > 1) && !(col && TPL == 1 && Z == 1 && NC <= 32);
   if (counted) unroll = false;
+  else if (col && cached.empty()) unroll = true;  // a thread per short line: its loads go out together
   // with caches, later phases need fewer recomputations: rebuild need sets
   if (!cached.empty()) {
     need.assign(nph + 2, {});
@@ -1226,7 +1241,7 @@ void Gen::emit_partials(int ni) {
 void Gen::emit_head(const std::string& entry) {
   o << "extern \"C\" __global__ void __launch_bounds__(" << WG << ") ";
   // line kernels: ask for the occupancy the cache budget was sized for (two groups per CU)
-  if (!flat && min_waves > 1 && !counted) o << "__attribute__((amdgpu_waves_per_eu(" << min_waves << "))) ";
+  if (!flat && min_waves > 1 && !(cached.empty() && (col || Z > 1))) o << "__attribute__((amdgpu_waves_per_eu(" << min_waves << "))) ";
   o << entry << "(";
   for (size_t i = 0; i < param_slots.size(); ++i) o << (i ? ", " : "") << "void* __restrict__ p" << i;
   if (mode != WHOLE) o << (param_slots.empty() ? "" : ", ") << "u8* __restrict__ ps";

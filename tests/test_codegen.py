@@ -386,3 +386,14 @@ def test_rows_of_odd_length_take_whole_vectors_where_few_or_long(rows, cols, dt,
     kernel = g.codegen([y, g.argmax(y, 1)], compile=True).split("__global__")[1]
     assert int(re.search(r"float f0\[(\d+)\]", kernel).group(1)) == vector
     assert bool(re.search(r"if \(lane < \d+u\)", kernel)) == (vector == (4 if dt == DType.F32 else 8))  # the elements left over
+
+
+@pytest.mark.parametrize("op,shape,dt,lines,along", [
+    ("softmax", (16, 131072), DType.BF16, 1, 1), ("softmax", (16, 524288), DType.BF16, 8, 1), ("softmax", (16, 400000), DType.F32, 4, 1),
+    ("argmax", (2, 3000000), DType.BF16, 1, 1), ("argmax", (24, 8000), DType.F32, 1, 1), ("sum", (24, 8000), DType.F32, 4, 2)])
+def test_short_columns_take_lines_a_thread_where_they_fill_the_chip(op, shape, dt, lines, along):
+    g = Graph()
+    x = g.input(list(shape), dt)
+    kernel = g.codegen([getattr(g, op)(x, 0)], compile=True).split("__global__")[1]
+    threads, across = (int(re.search(p, kernel).group(1)) for p in (r"__launch_bounds__\((\d+)\)", r"lane = threadIdx\.x / (\d+)u"))
+    assert (int(re.search(r"float f0\[(\d+)\]", kernel).group(1)), threads // across) == (lines, along)

@@ -131,10 +131,11 @@ def test_reductions_of_no_lines_are_empty(hip, shape, axis):
     check(hip, g, [g.sum(x, axis), g.argmax(x, axis), y], {x: Tensor(DType.F32, shape, b"")}, f"no lines {shape} axis {axis}")
 
 
-# one to eight adjacent lines a thread, which take 16384 lines each: short columns with one thread a
-# line and their values in registers, long ones with up to 16 threads and 128 KB of LDS; a middle axis
-@pytest.mark.parametrize("shape,axis,dt", [((40, 32768), 0, DType.F32), ((12, 65536), 0, DType.F32), ((100, 65536), 0, DType.F32),
-                                           ((3, 30, 22000), 1, DType.F32), ((9, 131072), 0, DType.BF16), ((130, 131072), 0, DType.BF16),
+# one to eight adjacent lines a thread: short columns with one thread a line and their values in
+# registers (from 65536 such threads), long ones with up to 16 threads and 128 KB of LDS (from 16384); a
+# middle axis
+@pytest.mark.parametrize("shape,axis,dt", [((40, 32768), 0, DType.F32), ((12, 270000), 0, DType.F32), ((100, 65536), 0, DType.F32),
+                                           ((3, 30, 22000), 1, DType.F32), ((9, 600000), 0, DType.BF16), ((9, 131072), 0, DType.BF16), ((130, 131072), 0, DType.BF16),
                                            ((130, 131080), 0, DType.BF16)])
 def test_column_softmax_rmsnorm_and_argmax_of_many_lines_match_f64(hip, shape, axis, dt):
     """Several levels of reduction over several lines a thread. f32 at the bar of 1e-5; bf16 within one
