@@ -64,7 +64,9 @@ GemmRoute quant_flex_route(const QuantArgs& q) {
     // for f32 values, which go to LDS one by one
     const double extra = kTiles[i].bn * 64 * 4.5 / 64 / 2100;
     for (int64_t s = 1; s <= 64 && (s == 1 || kt / s >= 2); s *= 2) {
-      const double us = gemm_flex_cost(a, i, s, extra, b_bytes);
+      // Few stages of the 128 x 128 tile in 16 bits take 11 us before the first pays (int4 520 x 4096 x
+      // 192 14.0 us, on 64 x 64 tiles 7.8), not the 4 that gemm_flex_cost counts for all.
+      const double us = gemm_flex_cost(a, i, s, extra, b_bytes) + (i == 0 && !is32 && kt <= 8 ? 7 : 0);
       if (us < best.us) best = {GemmPath::FLEX, i, s, us};
     }
   }

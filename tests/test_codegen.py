@@ -397,3 +397,12 @@ def test_short_columns_take_lines_a_thread_where_they_fill_the_chip(op, shape, d
     kernel = g.codegen([getattr(g, op)(x, 0)], compile=True).split("__global__")[1]
     threads, across = (int(re.search(p, kernel).group(1)) for p in (r"__launch_bounds__\((\d+)\)", r"lane = threadIdx\.x / (\d+)u"))
     assert (int(re.search(r"float f0\[(\d+)\]", kernel).group(1)), threads // across) == (lines, along)
+
+
+@pytest.mark.parametrize("m,n,k,want", [(520, 4096, 192, "_fused"), (1000, 4096, 256, ""), (260, 4096, 4096, "_fused")])
+def test_quant_route_counts_the_large_tile_start(m, n, k, want):
+    g = Graph()
+    qw = g.constant_bytes(DType.U8, bytes(n * k // 2), [n, k // 2])
+    scales = g.constant_bytes(DType.F16, np.ones((n, k // 64), np.float16).tobytes(), [n, k // 64])
+    y = g.quant_matmul(g.input([m, k], DType.BF16), qw, scales, None, 4, 64)
+    assert [s.split()[0] for s in steps(g.codegen([y]))] == ["quant_dequant+gemm" + want]
