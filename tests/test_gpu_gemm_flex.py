@@ -150,6 +150,10 @@ def test_steps_of_a_plan_share_their_scratch():
     assert sum("_split" in s for s in labels) == count, labels
     plan.launch()
     got = [plan.output(i).numpy() for i in range(2 * count + 1)]
+    for _ in range(3):  # recorded, then replayed
+        plan.launch(use_graph=True)
+        for i, want in enumerate(got):
+            np.testing.assert_array_equal(plan.output(i).numpy(), want)
     np.testing.assert_array_equal(np.concatenate(got[:count]), a @ b)  # sums of few 64ths: exact in any order
     wq = np.stack([(q & 15).astype(np.int8), (q >> 4).astype(np.int8)], -1).reshape(n, k)
     wq = np.where(wq > 7, wq - 16, wq).astype(np.float32) * 0.25
